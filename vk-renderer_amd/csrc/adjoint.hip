@@ -65,7 +65,10 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(const AdjointLaunch A)
         __syncthreads();
     }
 
-    bool has = false, exhausted = false;
+    bool has = false;
+    const uint32_t lanes = gridDim.x * BLOCK;
+    ItemPool pool;
+    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     float uvx = 0.0f, uvy = 0.0f, salt = 0.0f, salt0 = 0.0f;
     uint32_t smp = 0, depth = 0, phase = kPhTrace, pass = MODE, zb = 0, nchain = 0, cstar = 0, hs = kMiss;
     uint32_t pix = 0;
@@ -134,25 +137,9 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(const AdjointLaunch A)
     };
 
     while (true) {
-        if (!exhausted) {
-            const unsigned long long need = __ballot(!has);
-            const unsigned long long busy = __ballot(has);
-            const uint32_t nneed = (uint32_t)__popcll(need);
-            if (nneed > 0 && (nneed >= 32u || busy == 0)) {
-                const int leader = __ffsll((long long)need) - 1;
-                uint32_t base = 0;
-                if (__lane_id() == leader) base = atomicAdd(cursor, nneed);
-                base = __shfl(base, leader, 64);
-                if (base + nneed >= A.total) exhausted = true;
-                if (!has) {
-                    const uint32_t rank = (uint32_t)__popcll(need & ((1ull << __lane_id()) - 1ull));
-                    const uint32_t g = base + rank;
-                    if (g < A.total) claim(g);
-                }
-            }
-        }
+        pool.refill(cursor, A.total, lanes, 32u, has, claim);
         if (__ballot(has) == 0) {
-            if (exhausted) break;
+            if (pool.dry) break;
             continue;
         }
 
@@ -417,7 +404,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(const AdjointLaunch A)
         }
     }
 
-    flush_counter(&A.counters->rays, c_rays);
+    flush_counter(&counter_bank(A.counters, blockIdx.x)->rays, c_rays);
     if (LDSGRAD) {
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < np; i += BLOCK)

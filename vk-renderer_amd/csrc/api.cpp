@@ -109,9 +109,9 @@ vkr_error vkr_create(const vkr_create_info* info, vkr_ctx** out_ctx)
     auto ctx = std::make_unique<vkr_ctx>();
     ctx->device = dev;
     ctx->flags = info ? info->flags : 0u;
-    VKR_HIP(ctx->counters.alloc(sizeof(DevCounters)));
+    VKR_HIP(ctx->counters.alloc(kCounterBanks * sizeof(DevCounters)));
     VKR_HIP(ctx->pool.alloc(64));
-    VKR_HIP(hipMemset(ctx->counters.p, 0, sizeof(DevCounters)));
+    VKR_HIP(hipMemset(ctx->counters.p, 0, kCounterBanks * sizeof(DevCounters)));
     // The device address of this device's static scratch (vkr_trace_frame_static).
     char* scratch = nullptr;
     VKR_HIP(static_scratch(dev, &scratch));
@@ -426,7 +426,7 @@ vkr_error vkr_trace_frame(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd
         if (ae != VKR_SUCCESS) return ae;
         j.adj_samples = ctx->adj_samples.as<uint2>();
     }
-    DevCounters* cnt = ctx->counters.as<DevCounters>();
+    const CounterRef cnt = banked(ctx->counters);
     uint32_t* pool = ctx->pool.as<uint32_t>();
     VKR_HIP(launch_zero_counters(cnt, pool, st));
     if (params->kernel == VKR_KERNEL_WHITTED) {
@@ -507,7 +507,7 @@ vkr_error vkr_trace_frame_static(vkr_ctx* ctx, uint32_t scene, const vkr_frame_d
     VKR_HIP(hipSetDevice(ctx->device));
     char* scratch = nullptr;
     VKR_HIP(static_scratch(ctx->device, &scratch));
-    DevCounters* cnt = reinterpret_cast<DevCounters*>(scratch);
+    const CounterRef cnt{reinterpret_cast<DevCounters*>(scratch), 0u};   // one bank: the static array is of fixed size
     uint32_t* pool = reinterpret_cast<uint32_t*>(scratch + kStaticPoolOff);
     char* lanes = scratch + kStaticLanesOff;
     const size_t max_lanes = (size_t)VKR_STATIC_SCRATCH_LANE_BYTES / kLaneBytes;
@@ -572,7 +572,7 @@ vkr_error vkr_trace_frame_static(vkr_ctx* ctx, uint32_t scene, const vkr_frame_d
     }
     ctx->timed = false;
     ctx->last_static = true;
-    ctx->last_counters = cnt;
+    ctx->last_counters = cnt.banks;
     return VKR_SUCCESS;
 }
 
@@ -582,9 +582,16 @@ vkr_error vkr_last_counters(vkr_ctx* ctx, vkr_counters* out)
     VKR_HIP(hipSetDevice(ctx->device));
     if (ctx->timed) VKR_HIP(hipEventSynchronize(ctx->ev1));
     if (ctx->last_static) VKR_HIP(hipDeviceSynchronize());   // that call recorded no events
-    DevCounters c{};
     const void* src = ctx->last_counters ? (const void*)ctx->last_counters : ctx->counters.p;
-    VKR_HIP(hipMemcpy(&c, src, sizeof(c), hipMemcpyDeviceToHost));
+    const uint32_t n = ctx->last_static ? 1u : kCounterBanks;
+    DevCounters banks[kCounterBanks], c{};
+    VKR_HIP(hipMemcpy(banks, src, n * sizeof(DevCounters), hipMemcpyDeviceToHost));
+    for (uint32_t i = 0; i < n; ++i) {
+        const DevCounters& b = banks[i];
+        c.rays += b.rays; c.shadow += b.shadow; c.traced += b.traced; c.nodes += b.nodes;
+        c.tris += b.tris; c.spheres += b.spheres; c.planes += b.planes; c.overflow += b.overflow;
+        c.wave_nodes += b.wave_nodes; c.wave_leaves += b.wave_leaves; c.wave_steps += b.wave_steps;
+    }
     out->rays = c.rays;
     out->shadow_rays = c.shadow;
     out->nodes_visited = c.nodes;
@@ -685,7 +692,7 @@ vkr_error vkr_adjoint(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd, co
     a.d_radiance = d_radiance;
     a.d_params = d_params;
     a.params = s->theta.as<float>();
-    a.counters = ctx->counters.as<DevCounters>();
+    a.counters = banked(ctx->counters);
     a.pool = ctx->pool.as<uint32_t>();
     a.total = a.job.n_tiles * 64u;
     // The second pass hands out one item per (pixel, sample) of whole tiles.

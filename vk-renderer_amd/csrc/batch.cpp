@@ -61,7 +61,7 @@ vkr_error plan_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, BatchP
 }
 
 PathLaunch batch_launch(const BatchPlan& plan, const JobDesc* djobs, const uint32_t* dstart, uint32_t n,
-                        uint32_t chunk, uint32_t* pool, DevCounters* cnt)
+                        uint32_t chunk, uint32_t* pool, CounterRef cnt)
 {
     PathLaunch a{};
     a.jobs = djobs;
@@ -88,9 +88,9 @@ uint32_t batch_grid(const BatchPlan& plan, const PathVariant& v, int device)
 
 bool valid_block(uint32_t b) { return b == 0 || b == 64 || b == 128 || b == 256; }
 
-// The 32-bit pool cursor: once the pool is empty, every resident wave that
-// has not yet seen it run dry still claims up to its 64 lanes' worth, so the
-// cursor can pass the total by at most the number of resident lanes.
+// The 32-bit item numbers: once the pool is empty, every resident wave that
+// has not yet seen it run dry still claims up to its 64 lanes' worth, so they
+// can pass the total by at most the number of resident lanes.
 vkr_error check_cursor(const BatchPlan& plan, uint32_t grid, uint32_t block)
 {
     if (plan.total + (uint64_t)grid * block > 0xFFFFFFFFull)
@@ -197,7 +197,7 @@ vkr_error vkr_trace_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n_jo
     VKR_HIP(hipMemcpyAsync(ctx->job_start.p, static_cast<char*>(ctx->host_jobs) + jb, sb, hipMemcpyHostToDevice, st));
     VKR_HIP(hipEventRecord(ctx->ev_copy, st));
 
-    DevCounters* cnt = ctx->counters.as<DevCounters>();
+    const CounterRef cnt = banked(ctx->counters);
     uint32_t* pool = ctx->pool.as<uint32_t>();
     const bool count = (ctx->flags & VKR_CTX_COUNT_WORK) != 0;
     const BatchShape sh = batch_shape(ctx, jobs, n_jobs, plan, block, chunk);
@@ -242,13 +242,13 @@ vkr_error vkr_batch_graph_create(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32
     VKR_HIP(g->jobs.upload(plan.jobs.data(), plan.jobs.size() * sizeof(JobDesc)));
     VKR_HIP(g->job_start.upload(plan.start.data(), plan.start.size() * sizeof(uint32_t)));
     VKR_HIP(g->pool.alloc(64));
-    VKR_HIP(g->counters.alloc(sizeof(DevCounters)));
+    VKR_HIP(g->counters.alloc(kCounterBanks * sizeof(DevCounters)));
     g->total = plan.total;
     g->n_jobs = n_jobs;
     g->job_scene.resize(n_jobs);
     for (uint32_t i = 0; i < n_jobs; ++i) g->job_scene[i] = jobs[i].scene;
     PathLaunch a = batch_launch(plan, g->jobs.as<JobDesc>(), g->job_start.as<uint32_t>(), n_jobs, sh.chunk,
-                                g->pool.as<uint32_t>(), g->counters.as<DevCounters>());
+                                g->pool.as<uint32_t>(), banked(g->counters));
     if (v.pool) {
         VKR_HIP(g->lanes.alloc((size_t)grid * sh.block * kLaneBytes));   // the graph's own records
         a.lanes = g->lanes.as<char>();
@@ -260,7 +260,7 @@ vkr_error vkr_batch_graph_create(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32
     VKR_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
     hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
-        const hipError_t e1 = launch_zero_counters(g->counters.as<DevCounters>(), g->pool.as<uint32_t>(), cap);
+        const hipError_t e1 = launch_zero_counters(banked(g->counters), g->pool.as<uint32_t>(), cap);
         const hipError_t e2 = launch_path(a, v, grid, cap);
         e = hipStreamEndCapture(cap, &g->graph);
         if (e == hipSuccess && e1 != hipSuccess) e = e1;

@@ -254,6 +254,9 @@ inline JobDesc make_job(const Scene& sc, const vkr_frame_data& fd, const vkr_tra
     return j;
 }
 
+// The counters of a buffer that holds kCounterBanks banks.
+inline CounterRef banked(const DevBuf& b) { return CounterRef{b.as<DevCounters>(), kCounterBanks - 1u}; }
+
 inline vkr_error ensure_events(vkr_ctx* ctx)
 {
     if (!ctx->ev0) VKR_HIP(hipEventCreate(&ctx->ev0));

@@ -54,9 +54,19 @@ struct JobDesc {
                                   // sample's start, clamp-saturation bits) for the adjoint; NULL: none
 };
 
-struct DevCounters {
+// Atomics on one address are served one after the other, 11.5 ns each
+// whatever the number of waves; on 64 lines they take 0.4 ns each.  So a
+// launch counts into kCounterBanks copies of the counters, one cache line
+// each (a workgroup adds to bank blockIdx % banks), and the host sums them.
+struct alignas(128) DevCounters {
     unsigned long long rays, shadow, traced, nodes, tris, spheres, planes, overflow;
     unsigned long long wave_nodes, wave_leaves, wave_steps;
+};
+constexpr uint32_t kCounterBanks = 64u;   // a power of two
+static_assert(sizeof(DevCounters) == 128, "one bank per 128-byte line");
+struct CounterRef {
+    DevCounters* banks;
+    uint32_t mask;                // number of banks - 1
 };
 
 // Default pool refill threshold: a wave claims new pixels once at least this
@@ -66,8 +76,9 @@ constexpr uint32_t kDefaultChunk = 8u;
 
 // Most work items one launch's 32-bit pool cursor hands out.  A resident
 // wave can add up to 64 to the cursor after the last item has gone (its one
-// claim that finds the pool empty), so the cursor stays below 2^32 while the
-// resident lanes number under 2^24.
+// claim that finds the pool empty), and items are numbered from the resident
+// lanes up, so the numbers stay below 2^32 while the resident lanes number
+// under 2^23.
 constexpr uint64_t kMaxPoolItems = 0xFF000000ull;
 
 // One-pixel-per-lane launches cover at most this many lanes each, which
@@ -115,7 +126,7 @@ struct PathLaunch {
     uint32_t base;                // one pixel per lane: pool index of the launch's lane 0
     uint32_t chunk;               // refill when at least this many lanes idle
     uint32_t* pool;               // persistent pool cursor (device)
-    DevCounters* counters;
+    CounterRef counters;
     char* lanes;                  // ray records: one kWaveBytes block per wave of the grid
 };
 
@@ -125,7 +136,7 @@ struct AdjointLaunch {
     const float* d_radiance;      // W*H*4
     float* d_params;              // 7 * n_spheres + 1
     const float* params;          // 7 * n_spheres + 1 (current values)
-    DevCounters* counters;
+    CounterRef counters;
     uint32_t* pool;               // persistent pool cursors: [0] pass 1, [1] pass 2
     uint32_t total;               // pool indices (64 per 8x8 tile; pass 2: per tile and sample)
     uint2* samples;               // W*H*spp: (bits of the random-stream position at the sample's
@@ -141,13 +152,13 @@ struct PathVariant {
 };
 
 hipError_t launch_path(const PathLaunch& a, const PathVariant& v, uint32_t grid, hipStream_t s);
-hipError_t launch_whitted(const JobDesc& j, DevCounters* c, hipStream_t s);
+hipError_t launch_whitted(const JobDesc& j, CounterRef c, hipStream_t s);
 hipError_t launch_filter(const uint8_t* cur, const uint8_t* prev, uint32_t sw, uint32_t sh, uint8_t* out,
                          uint32_t dw, uint32_t dh, hipStream_t s);
 // pass1 false: a.samples already holds the first pass's records of this frame.
 hipError_t launch_adjoint(const AdjointLaunch& a, uint32_t stack, bool pass1, hipStream_t s);
 hipError_t launch_debug(uint32_t op, const float* in, float* out, uint32_t n, hipStream_t s);
-hipError_t launch_zero_counters(DevCounters* c, uint32_t* pool, hipStream_t s);
+hipError_t launch_zero_counters(CounterRef c, uint32_t* pool, hipStream_t s);
 // Writes the per-frame fields of a job in a device job table (camera,
 // aspect, seed, light position), in stream order.
 hipError_t launch_set_frame(JobDesc* job, const vkr_frame_data& fd, hipStream_t s);

@@ -181,7 +181,9 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
 
     // Lane state.
     bool has = false;
-    bool exhausted = !A.persistent;
+    const uint32_t lanes = gridDim.x * BLOCK;
+    ItemPool pool;
+    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + (wbase >> 6));
     uint32_t job = 0, px = 0, py = 0;
     float uvx = 0.0f, uvy = 0.0f, salt = 0.0f;
     uint32_t smp = 0, depth = 0, phase = kPhTrace;
@@ -235,26 +237,10 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
     }
 
     while (true) {
-        if (A.persistent && !exhausted) {
-            const unsigned long long need = __ballot(!has);
-            const unsigned long long busy = __ballot(has);
-            const uint32_t nneed = (uint32_t)__popcll(need);
-            if (nneed > 0 && (nneed >= A.chunk || busy == 0)) {
-                const int leader = __ffsll((long long)need) - 1;
-                uint32_t base = 0;
-                if (__lane_id() == leader) base = atomicAdd(A.pool, nneed);
-                base = __shfl(base, leader, 64);
-                if (base + nneed >= A.total) exhausted = true;
-                if (!has) {
-                    const uint32_t rank = (uint32_t)__popcll(need & ((1ull << __lane_id()) - 1ull));
-                    const uint32_t g = base + rank;
-                    if (g < A.total) claim(g);
-                }
-            }
-        }
+        if (A.persistent) pool.refill(A.pool, A.total, lanes, A.chunk, has, claim);
         const unsigned long long live = __ballot(has);
         if (live == 0) {
-            if (exhausted) break;
+            if (!A.persistent || pool.dry) break;
             continue;
         }
         if (COUNT && __lane_id() == 0) ++wave_steps;
@@ -650,18 +636,19 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
         }
     }
 
-    flush_counter(&A.counters->rays, c_rays);
-    flush_counter(&A.counters->shadow, c_shadow);
-    flush_counter(&A.counters->traced, c_traced);
-    flush_counter(&A.counters->overflow, wc.overflow);
+    DevCounters* const cnt = counter_bank(A.counters, blockIdx.x);
+    flush_counter(&cnt->rays, c_rays);
+    flush_counter(&cnt->shadow, c_shadow);
+    flush_counter(&cnt->traced, c_traced);
+    flush_counter(&cnt->overflow, wc.overflow);
     if (COUNT) {
-        flush_counter(&A.counters->nodes, wc.nodes);
-        flush_counter(&A.counters->tris, wc.tris);
-        flush_counter(&A.counters->spheres, wc.spheres);
-        flush_counter(&A.counters->planes, wc.planes);
-        flush_counter(&A.counters->wave_nodes, wc.wave_nodes);
-        flush_counter(&A.counters->wave_leaves, wc.wave_leaves);
-        flush_counter(&A.counters->wave_steps, wave_steps);
+        flush_counter(&cnt->nodes, wc.nodes);
+        flush_counter(&cnt->tris, wc.tris);
+        flush_counter(&cnt->spheres, wc.spheres);
+        flush_counter(&cnt->planes, wc.planes);
+        flush_counter(&cnt->wave_nodes, wc.wave_nodes);
+        flush_counter(&cnt->wave_leaves, wc.wave_leaves);
+        flush_counter(&cnt->wave_steps, wave_steps);
     }
 }
 
@@ -793,7 +780,7 @@ __device__ C4 render(const JobDesc& j, f3& ro, f3& rd, uint32_t& bounce, uint32_
 }
 }  // namespace whitted
 
-__global__ __launch_bounds__(256) void k_whitted(const JobDesc j, DevCounters* counters)
+__global__ __launch_bounds__(256) void k_whitted(const JobDesc j, CounterRef counters)
 {
     const uint32_t x = blockIdx.x * 16u + (threadIdx.x & 15u);
     const uint32_t y = blockIdx.y * 16u + (threadIdx.x >> 4);
@@ -828,8 +815,9 @@ __global__ __launch_bounds__(256) void k_whitted(const JobDesc j, DevCounters* c
         if (j.hit_t) j.hit_t[pi] = pt;
         if (j.ray_count) j.ray_count[pi] = rays;
     }
-    flush_counter(&counters->rays, rays);
-    flush_counter(&counters->traced, rays);
+    DevCounters* const cnt = counter_bank(counters, blockIdx.y * gridDim.x + blockIdx.x);
+    flush_counter(&cnt->rays, rays);
+    flush_counter(&cnt->traced, rays);
 }
 
 // ---------------------------------------------------------------------------
@@ -932,16 +920,12 @@ __global__ __launch_bounds__(256) void k_debug(uint32_t op, const float* in, flo
     }
 }
 
-__global__ void k_zero(DevCounters* c, uint32_t* pool)
+__global__ __launch_bounds__(256) void k_zero(CounterRef c, uint32_t* pool)
 {
-    if (threadIdx.x == 0) {
-        c->rays = c->shadow = c->traced = c->nodes = c->tris = c->spheres = c->planes = c->overflow = 0ull;
-        c->wave_nodes = c->wave_leaves = c->wave_steps = 0ull;
-        if (pool) {
-            pool[0] = 0u;
-            pool[1] = 0u;   // the adjoint's second pass
-        }
-    }
+    unsigned long long* w = reinterpret_cast<unsigned long long*>(c.banks);
+    const uint32_t n = (c.mask + 1u) * (uint32_t)(sizeof(DevCounters) / sizeof(unsigned long long));
+    for (uint32_t i = threadIdx.x; i < n; i += 256u) w[i] = 0ull;
+    if (pool && threadIdx.x < 2u) pool[threadIdx.x] = 0u;   // [1]: the adjoint's second pass
 }
 
 // ---------------------------------------------------------------------------
@@ -1010,7 +994,7 @@ uint32_t persistent_grid(const PathVariant& v, int device)
     return grid;
 }
 
-hipError_t launch_whitted(const JobDesc& j, DevCounters* c, hipStream_t s)
+hipError_t launch_whitted(const JobDesc& j, CounterRef c, hipStream_t s)
 {
     hipLaunchKernelGGL(k_whitted, dim3((j.W + 15) / 16, (j.H + 15) / 16), dim3(256), 0, s, j, c);
     return hipGetLastError();
@@ -1078,9 +1062,9 @@ hipError_t static_scratch(int device, char** out)
     return hipSuccess;
 }
 
-hipError_t launch_zero_counters(DevCounters* c, uint32_t* pool, hipStream_t s)
+hipError_t launch_zero_counters(CounterRef c, uint32_t* pool, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, s, c, pool);
+    hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, s, c, pool);
     return hipGetLastError();
 }
 

@@ -449,6 +449,56 @@ __device__ __forceinline__ void flush_counter(unsigned long long* dst, uint32_t 
     if (__lane_id() == 0 && s) atomicAdd(dst, (unsigned long long)s);
 }
 
+// The workgroup's copy of the launch's counters.
+__device__ __forceinline__ DevCounters* counter_bank(const CounterRef& c, uint32_t block)
+{
+    return c.banks + (block & c.mask);
+}
+
+// A wave's view of a launch's pool of work items.  The wave starts with the 64
+// items of its own number; the pool's cursor counts from the grid's lanes up,
+// so the waves of a launch do not open it with a queue of atomics on one
+// address (11.5 ns each).  Later claims take just the idle lanes' items: a
+// wave that kept a run of items to itself (a share of what is left, up to 64)
+// made fewer claims but left waves idle at the end of the launch while others
+// still held items (1080p heightfield 9.0 -> 11.5 ms, 1024^2 reference scene
+// 2.06 -> 2.50 ms).
+struct ItemPool {
+    uint32_t own;             // first of the wave's own items (kNoItem: taken)
+    bool dry;                 // nothing is left behind the cursor
+    static constexpr uint32_t kNoItem = 0xFFFFFFFFu;
+
+    __device__ __forceinline__ void start(uint32_t wave)
+    {
+        own = wave * 64u;
+        dry = false;
+    }
+    // Gives items to the idle lanes (has == false) once at least `chunk` of
+    // them wait: claim(item) for each.  Every lane of the wave calls it.
+    template <class Claim>
+    __device__ __forceinline__ void refill(uint32_t* cursor, uint32_t total, uint32_t lanes, uint32_t chunk, bool has,
+                                           Claim&& claim)
+    {
+        const unsigned long long need = __ballot(!has);
+        const uint32_t n = (uint32_t)__popcll(need);
+        if (n == 0u || n < chunk || dry) return;
+        uint32_t base = own;
+        if (own == kNoItem) {
+            base = 0u;
+            if (__lane_id() == 0) base = atomicAdd(cursor, n);
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + lanes;
+        }
+        own = kNoItem;
+        // (Items below `lanes` are the waves' own: a wave whose own items lie
+        // past the total finds the cursor's there too.)
+        dry = base + n >= total && base >= lanes;
+        if (!has) {
+            const uint32_t g = base + (uint32_t)__popcll(need & ((1ull << __lane_id()) - 1ull));
+            if (g < total) claim(g);
+        }
+    }
+};
+
 // XCD-aware remap: consecutive workgroup ids land on different XCDs, so give
 // each XCD a contiguous range of tiles (its L2 then sees neighbouring rays).
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t g)

@@ -89,30 +89,33 @@ constexpr uint32_t kMaxPlainLanes = 1u << 21;
 // kWaveBytes per wave (64 lanes), laid out field by field so that the lanes
 // of a wave reading or writing one field touch contiguous addresses.  Field
 // f of lane l is at f + 16 l; per-slot fields hold slot k of lane l at
-// f + 16 (64 k + l) (salts: f + 4 (64 k + l)).
-//   kWPark   4 x float4: path state parked while the wave traces
-//            (ro, dj.x) (rd, dj.y) (P, dj.z) (N, 0), at kWPark + 1024 i
-//   kWHead   this step's ray origin xyz; w holds the bits of (job << 1) | 1
-//            for shadow rays, (job << 1) for a closest-hit ray (job: index
-//            in the batch, 0 for a single frame)
-//   kWSlotD  per slot: the ray's (d xyz, t_max); slot k holds emitter
-//            ei0 + k of a next-event window, or slot 0 the path segment
-//   kWSlotC  per slot: the next-event contribution (xyz, 0)
+// f + 16 (64 k + l) (salts: f + 4 (64 k + l)).  Slot 0 is the path segment,
+// slots 1.. are emitters ei0 + k - 1 of a next-event window.
+//   kWPark   4 x float4: path state parked while the wave evaluates and
+//            traces (acc, u) (mask, v) (e, random-stream position) and, once
+//            per pixel, (bits of the primary hit's primitive, its t, -, -),
+//            at kWPark + 1024 i
+//   kWHead   the origin xyz of this step's rays; w holds the bits of the job
+//            (index in the batch, 0 for a single frame)
+//   kWSlotD  per slot: the ray's (d xyz, t_max)
+//   kWSlotC  per slot: the next-event contribution (xyz, 0); slot 0 (a
+//            segment has none) holds kWPix, the sum of the pixel's finished
+//            samples (xyz)
 //   kWHit    3 x float4: the diffuse hit published for the wave's
 //            next-event evaluation: (N xyz, u), (albedo xyz, roughness),
 //            (metalness, v, bits of ei0, bits of the kNee* flags)
-//   kWSalt   per slot: the random stream position before emitter ei0 + k's
+//   kWSalt   per slot: the random stream position before that emitter's
 //            sample
-//   kWPix    the sum of the pixel's finished samples (xyz)
 constexpr uint32_t kRaySlots = 32;
+constexpr uint32_t kNeeSlots = kRaySlots - 1u;   // emitters of one window
 constexpr uint32_t kWPark = 0u;
 constexpr uint32_t kWHead = kWPark + 4u * 1024u;
 constexpr uint32_t kWSlotD = kWHead + 1024u;
 constexpr uint32_t kWSlotC = kWSlotD + kRaySlots * 1024u;
+constexpr uint32_t kWPix = kWSlotC;
 constexpr uint32_t kWHit = kWSlotC + kRaySlots * 1024u;
 constexpr uint32_t kWSalt = kWHit + 3u * 1024u;
-constexpr uint32_t kWPix = kWSalt + kRaySlots * 256u;
-constexpr uint32_t kWaveBytes = kWPix + 1024u;
+constexpr uint32_t kWaveBytes = kWSalt + kRaySlots * 256u;
 constexpr uint32_t kLaneBytes = kWaveBytes / 64u;   // what one lane of a launch needs
 static_assert(kWaveBytes % 64u == 0u, "a wave's records split evenly over its lanes");
 

@@ -318,6 +318,59 @@ __device__ __forceinline__ TravOut traverse(const DevScene& sc, f3 o, f3 d, floa
     return r.finish<COUNT>(sc, eps, wc);
 }
 
+// Whether a plane stops a shadow ray (the tests of Ray::finish; their order
+// does not matter to a yes or no).
+template <bool COUNT>
+__device__ __forceinline__ bool plane_stops(const DevScene& sc, f3 o, f3 d, float tmax, float eps, WorkCnt& wc)
+{
+    const vkr_plane* __restrict__ planes = sc.planes;
+    for (uint32_t i = 0; i < sc.n_planes; ++i) {
+        if (COUNT) wc.planes++;
+        const float t = plane_t(o, d, ld3(planes[i].N), planes[i].len);
+        if ((t > eps) && (t < tmax - eps)) return true;
+    }
+    return false;
+}
+
+// Up to two rays per lane from one origin: a shadow ray (sh: direction sd,
+// length st) and the path segment that leaves the same point (seg: direction
+// d, t_max).  A lane whose shadow ray ends goes on with its segment while
+// other lanes still trace, so the wave waits for its longest sum of two rays
+// and not for two longest rays.  The shadow ray's planes come first: all
+// lanes test them together, and a ray they stop is not traversed.
+template <int BLOCK, bool COUNT>
+__device__ __forceinline__ TravOut traverse_pair(const DevScene& sc, f3 o, bool sh, f3 sd, float st, bool seg, f3 d,
+                                                 float tmax, float eps, uint32_t* stk, WorkCnt& wc, bool& occluded)
+{
+    occluded = sh && plane_stops<COUNT>(sc, o, sd, st, eps, wc);
+    const bool first = sh && !occluded;
+    bool next = first && seg;   // a segment waits behind the shadow ray
+    Ray r;
+    r.start(sc, o, first ? sd : d, first ? st : tmax, eps, first);
+    stk[0] = kDone;
+    if (!first && !seg) r.ref = kDone;
+    while (true) {
+        if (next && r.ref == kDone) {
+            occluded = r.occluded;
+            r.start(sc, o, d, tmax, eps, false);
+            next = false;
+        }
+        while (true) {
+            const uint32_t nn = (uint32_t)__popcll(__ballot((int)r.ref >= 0));
+            const uint32_t nw = (uint32_t)__popcll(__ballot((int)r.ref < -1 || (next && r.ref == kDone)));
+            if (leave_nodes(nn, nw)) break;
+            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(sc.nodes, stk, wc);
+            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(sc.nodes, stk, wc);
+        }
+        if (__ballot(r.ref != kDone || next) == 0) break;
+        if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(sc, eps, stk, wc);
+    }
+    if (r.any) occluded = r.occluded;   // a shadow ray with no segment behind it
+    if (!seg) return TravOut{kMiss, tmax, false};
+    r.any = false;
+    return r.finish<COUNT>(sc, eps, wc);
+}
+
 constexpr uint32_t kNone = 0xFFFFu;
 
 // Numbers a wave's work items slot by slot: `bits` holds the slots this lane
@@ -375,9 +428,9 @@ __device__ __forceinline__ void pool_item(const uint32_t* cpre, const unsigned l
 // 0..total of the wave until none is left, so a step costs the wave's total
 // work plus the last rays' tail instead of its longest lane.  Rays are
 // numbered slot by slot: rays cpre[k] .. cpre[k+1]-1 are slot k of the lanes
-// whose bit is set in colm[k], in lane order.  A shadow ray sets bit `slot`
-// of occ[owner] when occluded; the closest-hit ray of lane `owner` writes
-// (prim, t) to res[owner].  `wrec` is the wave's block of ray records
+// whose bit is set in colm[k], in lane order.  Slot 0 is the path segment of
+// lane `owner`, which writes (prim, t) to res[owner]; the others are shadow
+// rays, which set bit `slot` of occ[owner] when occluded.  `wrec` is the wave's block of ray records
 // (kWHead, kWSlotD: the lanes of a wave reading one slot of neighbouring
 // owners read neighbouring addresses).
 template <int BLOCK, bool COUNT, bool BATCH>
@@ -416,9 +469,8 @@ __device__ __forceinline__ void traverse_pool(const JobDesc* jobs, uint32_t tota
                     cur = (lo << 5) | slot;
                     const float4 h = *reinterpret_cast<const float4*>(wrec + (kWHead + lo * 16u));
                     const float4 s = *reinterpret_cast<const float4*>(wrec + (kWSlotD + (slot * 64u + lo) * 16u));
-                    const uint32_t hw = __float_as_uint(h.w);   // (owner's job << 1) | shadow ray
-                    if constexpr (BATCH) rj = jobs + (hw >> 1);
-                    r.start(rj->sc, f3{h.x, h.y, h.z}, f3{s.x, s.y, s.z}, s.w, rj->eps, (hw & 1u) != 0u);
+                    if constexpr (BATCH) rj = jobs + __float_as_uint(h.w);   // the owner's job
+                    r.start(rj->sc, f3{h.x, h.y, h.z}, f3{s.x, s.y, s.z}, s.w, rj->eps, slot != 0u);
                 }
                 next += (uint32_t)__popcll(want);
             }

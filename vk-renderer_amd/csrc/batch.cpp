@@ -75,9 +75,11 @@ PathLaunch batch_launch(const BatchPlan& plan, const JobDesc* djobs, const uint3
     return a;
 }
 
+// A batch of one job (the facade's captured frames) runs the single-frame
+// kernel on the job table: its job is uniform over the grid.
 PathVariant batch_variant(const BatchPlan& plan, uint32_t block, bool count)
 {
-    return PathVariant{block, plan.stack, count, true, plan.pool};
+    return PathVariant{block, plan.stack, count, plan.jobs.size() > 1u, plan.pool};
 }
 
 uint32_t batch_grid(const BatchPlan& plan, const PathVariant& v, int device)
@@ -152,7 +154,7 @@ BatchShape batch_shape(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, Batc
     if (!s.block) s.block = 128u;
     if (!s.chunk) s.chunk = kDefaultChunk;
     if (!tuned && plan.stack == 24u && plan.tree_depth <= 8u) {
-        const PathVariant v4{s.block, 32u, false, true, plan.pool};
+        const PathVariant v4{s.block, 32u, false, plan.jobs.size() > 1u, plan.pool};
         const uint64_t resident4 = (uint64_t)persistent_grid(v4, ctx->device) * s.block;
         plan.stack = plan.total <= resident4 ? 64u : 32u;
     }

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/vkr.h"
@@ -101,9 +102,10 @@ constexpr uint32_t kMaxPlainLanes = 1u << 21;
 //   kWSlotC  per slot: the next-event contribution (xyz, 0); slot 0 (a
 //            segment has none) holds kWPix, the sum of the pixel's finished
 //            samples (xyz)
-//   kWHit    3 x float4: the diffuse hit published for the wave's
+//   kWHit    4 x float4: the diffuse hit published for the wave's
 //            next-event evaluation: (N xyz, u), (albedo xyz, roughness),
-//            (metalness, v, bits of ei0, bits of the kNee* flags)
+//            (V xyz, metalness), (bits of the kNee* flags, v, bits of ei0, -);
+//            V = normalize(camera - P) is the same for every emitter
 //   kWSalt   per slot: the random stream position before that emitter's
 //            sample
 constexpr uint32_t kRaySlots = 32;
@@ -114,14 +116,14 @@ constexpr uint32_t kWSlotD = kWHead + 1024u;
 constexpr uint32_t kWSlotC = kWSlotD + kRaySlots * 1024u;
 constexpr uint32_t kWPix = kWSlotC;
 constexpr uint32_t kWHit = kWSlotC + kRaySlots * 1024u;
-constexpr uint32_t kWSalt = kWHit + 3u * 1024u;
+constexpr uint32_t kWSalt = kWHit + 4u * 1024u;
 constexpr uint32_t kWaveBytes = kWSalt + kRaySlots * 256u;
 constexpr uint32_t kLaneBytes = kWaveBytes / 64u;   // what one lane of a launch needs
 static_assert(kWaveBytes % 64u == 0u, "a wave's records split evenly over its lanes");
 
 struct PathLaunch {
-    JobDesc job;                  // single-frame launches
-    const JobDesc* jobs;          // batched launches
+    JobDesc job;                  // single-frame launches (first: the kernel finds it at its arguments' start)
+    const JobDesc* jobs;          // batched launches, and captured ones of one job; else NULL
     const uint32_t* job_start;    // n_jobs + 1 pool offsets (batched)
     uint32_t n_jobs;
     uint32_t total;               // pool indices (64 per 8x8 tile)
@@ -132,6 +134,8 @@ struct PathLaunch {
     CounterRef counters;
     char* lanes;                  // ray records: one kWaveBytes block per wave of the grid
 };
+
+static_assert(offsetof(PathLaunch, job) == 0, "uniform_job reads it there");
 
 // Adjoint launch (path replay), see adjoint.hip.
 struct AdjointLaunch {

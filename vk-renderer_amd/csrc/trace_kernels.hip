@@ -130,16 +130,18 @@ __device__ __forceinline__ bool nee_sample(const JobDesc& j, const NeeHit& h, ui
 
     const f3 sP = ld3(S->P);
     const float sr = S->r;
-    tl = length(sub(sP, P)) - sr;
     const f3 l0 = sub(sP, P);
+    float dist;
+    const f3 w0 = normalize_len(l0, dist);
+    tl = dist - sr;
     const float cos_a_max = sqrtf(1.0f - gclamp(sr * sr / dot(l0, l0), 0.0f, 1.0f));
     const float cosa = gmix(cos_a_max, 1.0f, rng_next(salt, uvx, uvy));
     const float phi = kTwoPi * rng_next(salt, uvx, uvy);
-    L = jitter(l0, phi, sqrtf(1.0f - cosa * cosa), cosa);
+    L = jitter_w(w0, phi, sqrtf(1.0f - cosa * cosa), cosa);
 
     const float x = tl / sr + 1.0f;
     f3 att = divs(muls(ld3(S->mat.emissive), 1.0f), x * x);
-    att = divs(subs(att, kAttSub), kAttDiv);
+    att = mul_recip(subs(att, kAttSub), kd(kAttDivR));
     att = maxs(att, 0.0f);
     const f3 F0 = mix3(f3{0.04f, 0.04f, 0.04f}, h.alb, h.metal);
     const f3 H = normalize(add(V, L));
@@ -152,8 +154,20 @@ __device__ __forceinline__ bool nee_sample(const JobDesc& j, const NeeHit& h, ui
     const float denominator = 4.0f * gmax(dot(N, V), 0.0f) * gmax(dot(N, L), 0.0f);
     const f3 specular = divs(numerator, gmax(denominator, 0.001f));
     const float NdotL = gmax(dot(N, L), 0.0f);
-    c = muls(mul(add(divs(mul(kD, h.alb), kPi), specular), att), NdotL);
+    c = muls(mul(add(mul_recip(mul(kD, h.alb), kd(kPiR)), specular), att), NdotL);
     return !(c.x == 0.0f && c.y == 0.0f && c.z == 0.0f);
+}
+
+// The job of a launch that has one: A.jobs in device memory (a captured graph's,
+// whose frame data is replaced between replays) or A.job among the kernel's
+// arguments (PathLaunch starts with it).  Constant memory through scalar
+// loads; `at` is opaque, so a field is loaded where it is used and does not
+// sit in scalar registers across the whole loop (some 140 of them were
+// spilled).
+__device__ __forceinline__ const JobDesc& uniform_job(unsigned long long at)
+{
+    asm volatile("" : "+s"(at));
+    return *(const JobDesc*)reinterpret_cast<const __attribute__((address_space(4))) JobDesc*>(at);
 }
 
 // The path program of Assets/Tracer.comp:433-593 as a per-lane state machine.
@@ -192,6 +206,9 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
     // This lane's element of a one-per-lane field f is at wrec + (f + lo16):
     // a wave-uniform base and a 32-bit offset, one address form for all fields.
     const uint32_t lo16 = __lane_id() * 16u;
+
+    const unsigned long long job_at =
+        A.jobs ? (unsigned long long)A.jobs : (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
 
     // Lane state.
     bool has = false;
@@ -263,7 +280,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
             job = lo;
             local = g - A.job_start[lo];
         }
-        const JobDesc& j = BATCH ? A.jobs[job] : A.job;
+        const JobDesc& j = BATCH ? A.jobs[job] : uniform_job(job_at);
         const uint32_t tile = local >> 6, within = local & 63u;
         if (tile >= j.n_tiles) return;
         const uint32_t x = (tile % j.tiles_x) * 8u + (within & 7u);
@@ -304,7 +321,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
         }
         if (COUNT && __lane_id() == 0) ++wave_steps;
 
-        const JobDesc& j = BATCH ? A.jobs[job] : A.job;
+        const JobDesc& jq = BATCH ? A.jobs[job] : uniform_job(job_at);
 
         // (2) Next-event samples (:464-469) and their unoccluded
         // contributions (:475-502), evaluated before the shadow rays
@@ -321,14 +338,16 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
                 // emitters; the wave evaluates all (lane, emitter) pairs
                 // together below.  Each sample draws twice (:464-465), so
                 // the stream position before each one is known now.
-                const uint32_t w = min(kNeeSlots, j.sc.n_emitters - ei);
+                const uint32_t w = min(kNeeSlots, jq.sc.n_emitters - ei);
                 if (ei == 0u) {
+                    const f3 V = normalize(sub(ld3(jq.cam_pos), ro));
                     *reinterpret_cast<float4*>(wrec + (kWHit + lo16)) = make_float4(N.x, N.y, N.z, uvx);
                     *reinterpret_cast<float4*>(wrec + (kWHit + 1024u + lo16)) =
                         make_float4(hm->albedo[0], hm->albedo[1], hm->albedo[2], hm->roughness);
+                    *reinterpret_cast<float4*>(wrec + (kWHit + 2048u + lo16)) = make_float4(V.x, V.y, V.z, hm->metalness);
                 }
-                *reinterpret_cast<float4*>(wrec + (kWHit + 2048u + lo16)) =
-                    make_float4(hm->metalness, uvy, __uint_as_float(ei), __uint_as_float(nee_flags));
+                *reinterpret_cast<float4*>(wrec + (kWHit + 3072u + lo16)) =
+                    make_float4(__uint_as_float(nee_flags), uvy, __uint_as_float(ei), 0.0f);
                 float* sk = reinterpret_cast<float*>(wrec + (kWSalt + 256u + __lane_id() * 4u));
                 float sv = salt;
                 for (uint32_t k = 0; k < w; ++k) {
@@ -346,29 +365,29 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
                 NeeHit h;
                 h.P = ro;
                 h.N = N;
-                h.V = normalize(sub(ld3(j.cam_pos), ro));
+                h.V = normalize(sub(ld3(jq.cam_pos), ro));
                 h.alb = ld3(hm->albedo);
                 h.rough = hm->roughness;
                 h.metal = hm->metalness;
                 h.flags = nee_flags;
-                while (ei < j.sc.n_emitters) {
+                while (ei < jq.sc.n_emitters) {
                     const float s0 = salt;
                     salt = salt + 1.0f;              // the sample's two draws (:464-465)
                     salt = salt + 1.0f;
                     ++rays_px;
                     ++c_rays;
                     ++c_shadow;
-                    if (nee_sample(j, h, ei++, s0, uvx, uvy, sd, st, c0)) {
+                    if (nee_sample(jq, h, ei++, s0, uvx, uvy, sd, st, c0)) {
                         ++c_traced;
                         sh = true;
                         break;
                     }
                 }
             }
-            if (ei >= j.sc.n_emitters) {
+            if (ei >= jq.sc.n_emitters) {
                 // The vertex's last emitters: its next segment goes along.
-                term = roulette(j, mul(mask, ld3(hm->albedo)));
-                seg = !term && depth + 1u < j.max_depth;
+                term = roulette(jq, mul(mask, ld3(hm->albedo)));
+                seg = !term && depth + 1u < jq.max_depth;
                 if (seg) {
                     ++rays_px;
                     ++c_rays;
@@ -384,7 +403,8 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
         if constexpr (!POOL) {
             // (3) At most a shadow ray and a segment per lane, from registers.
             bool occluded;
-            tr = traverse_pair<BLOCK, COUNT>(j.sc, ro, sh, sd, st, has && seg, rd, tmax, j.eps, stk, wc, occluded);
+            const JobDesc& jt = BATCH ? A.jobs[job] : uniform_job(job_at);
+            tr = traverse_pair<BLOCK, COUNT>(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, stk, wc, occluded);
             if (sh && !occluded) e = add(e, c0);                     // :473, :502
         } else {
             // Path state that the wave's evaluation and tracing do not need
@@ -416,19 +436,20 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
                     const float4 h0 = *reinterpret_cast<const float4*>(wrec + (kWHit + oo));
                     const float4 h1 = *reinterpret_cast<const float4*>(wrec + (kWHit + 1024u + oo));
                     const float4 h2 = *reinterpret_cast<const float4*>(wrec + (kWHit + 2048u + oo));
+                    const float4 h3 = *reinterpret_cast<const float4*>(wrec + (kWHit + 3072u + oo));
                     const float sk = *reinterpret_cast<const float*>(wrec + (kWSalt + (k * 64u + lo) * 4u));
-                    const JobDesc& oj = BATCH ? A.jobs[__float_as_uint(hd.w)] : A.job;
+                    const JobDesc& oj = BATCH ? A.jobs[__float_as_uint(hd.w)] : uniform_job(job_at);
                     NeeHit h;
                     h.P = f3{hd.x, hd.y, hd.z};
                     h.N = f3{h0.x, h0.y, h0.z};
-                    h.V = normalize(sub(ld3(oj.cam_pos), h.P));
+                    h.V = f3{h2.x, h2.y, h2.z};
                     h.alb = f3{h1.x, h1.y, h1.z};
                     h.rough = h1.w;
-                    h.metal = h2.x;
-                    h.flags = __float_as_uint(h2.w);
+                    h.metal = h2.w;
+                    h.flags = __float_as_uint(h3.x);
                     f3 L, c;
                     float tl;
-                    if (nee_sample(oj, h, __float_as_uint(h2.z) + k - 1u, sk, h0.w, h2.y, L, tl, c)) {
+                    if (nee_sample(oj, h, __float_as_uint(h3.z) + k - 1u, sk, h0.w, h3.y, L, tl, c)) {
                         const uint32_t so = (k * 64u + lo) * 16u;
                         *reinterpret_cast<float4*>(wrec + (kWSlotD + so)) = make_float4(L.x, L.y, L.z, tl);
                         *reinterpret_cast<float4*>(wrec + (kWSlotC + so)) = make_float4(c.x, c.y, c.z, 0.0f);
@@ -453,7 +474,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            traverse_pool<BLOCK, COUNT, BATCH>(BATCH ? A.jobs : &A.job, nrays, s_cpre + wslot, s_colm + wslot,
+            traverse_pool<BLOCK, COUNT, BATCH>(BATCH ? A.jobs : &uniform_job(job_at), nrays, s_cpre + wslot, s_colm + wslot,
                                                s_occ + wbase, s_res + wbase, wrec, stk, wc);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -486,6 +507,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
         if (!has) continue;
 
         // (4) End of a diffuse vertex (:507-511) and of its roulette.
+        const JobDesc& j = BATCH ? A.jobs[job] : uniform_job(job_at);
         bool path_end = ended;
         ended = false;
         if (nee) {

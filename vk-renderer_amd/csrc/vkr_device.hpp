@@ -28,6 +28,17 @@ struct f3 {
     float x, y, z;
 };
 
+// A double constant, put into scalar registers where it is used.  Otherwise
+// the compiler keeps the constants of every polynomial in vector registers
+// across the caller's whole loop (26 of them in the path kernel) and copies
+// each one before the multiply-add that takes it as its addend.
+__device__ __forceinline__ double kd(double c)
+{
+    unsigned long long b = __builtin_bit_cast(unsigned long long, c);
+    asm volatile("" : "+s"(b));
+    return __builtin_bit_cast(double, b);
+}
+
 __device__ __forceinline__ f3 mk(float x, float y, float z) { return f3{x, y, z}; }
 __device__ __forceinline__ f3 ld3(const float* p) { return f3{p[0], p[1], p[2]}; }
 __device__ __forceinline__ f3 add(f3 a, f3 b) { return f3{a.x + b.x, a.y + b.y, a.z + b.z}; }
@@ -35,7 +46,28 @@ __device__ __forceinline__ f3 sub(f3 a, f3 b) { return f3{a.x - b.x, a.y - b.y, 
 __device__ __forceinline__ f3 mul(f3 a, f3 b) { return f3{a.x * b.x, a.y * b.y, a.z * b.z}; }
 __device__ __forceinline__ f3 divv(f3 a, f3 b) { return f3{a.x / b.x, a.y / b.y, a.z / b.z}; }
 __device__ __forceinline__ f3 muls(f3 a, float s) { return f3{a.x * s, a.y * s, a.z * s}; }
-__device__ __forceinline__ f3 divs(f3 a, float s) { return f3{a.x / s, a.y / s, a.z / s}; }
+// Quotients a / b of three floats by one, each rounded as a float division
+// rounds it: (float)((double)a * r) with r = 1/b to within 2^-52.  A quotient
+// of two floats is at least 2^-49 (relative) away from any midpoint of two
+// floats, and r and the product are off by less than 2^-51 together, so the
+// rounding cannot differ; zeros, infinities, NaN and results below 2^-126
+// come out as a division gives them too.  Three divisions cost 131 cycles of
+// a SIMD, this 87; by a constant 142 and 43.
+__device__ __forceinline__ f3 mul_recip(f3 a, double r)
+{
+    return f3{(float)((double)a.x * r), (float)((double)a.y * r), (float)((double)a.z * r)};
+}
+constexpr int kZeroOrInf = 0x264;   // floating-point classes +-0 and +-infinity
+// y = 1/b or 1/sqrt to about 2^-22, refined with its residual e = 1 - by:
+// 1/b = y (1 + e + e^2 + ...).
+__device__ __forceinline__ double refine(double y, double e) { return __builtin_fma(__builtin_fma(e, e, e), y, y); }
+__device__ __forceinline__ double recip_d(float b)
+{
+    const double bd = (double)b;
+    const double y = __builtin_amdgcn_rcp(bd);
+    return __builtin_isfpclass(b, kZeroOrInf) ? y : refine(y, __builtin_fma(-bd, y, 1.0));
+}
+__device__ __forceinline__ f3 divs(f3 a, float s) { return mul_recip(a, recip_d(s)); }
 __device__ __forceinline__ f3 adds(f3 a, float s) { return f3{a.x + s, a.y + s, a.z + s}; }
 __device__ __forceinline__ f3 subs(f3 a, float s) { return f3{a.x - s, a.y - s, a.z - s}; }
 __device__ __forceinline__ f3 ssub(float s, f3 a) { return f3{s - a.x, s - a.y, s - a.z}; }
@@ -45,7 +77,30 @@ __device__ __forceinline__ f3 cross(f3 a, f3 b)
     return f3{a.y * b.z - b.y * a.z, a.z * b.x - b.z * a.x, a.x * b.y - b.x * a.y};
 }
 __device__ __forceinline__ float length(f3 a) { return sqrtf(dot(a, a)); }
-__device__ __forceinline__ f3 normalize(f3 a) { return divs(a, length(a)); }
+// v / length(v), and the length: the root as two steps of g += (x - g^2) / (2
+// sqrt x) in double, whose error (2^-53) is below the least distance of a
+// float's root from a midpoint (2^-51), then the quotients as in divs with
+// the reciprocal refined from the same 1/sqrt estimate.  230 cycles of a SIMD
+// with a float root and three divisions, this 147.
+__device__ __forceinline__ f3 normalize_len(f3 a, float& len)
+{
+    const float x = dot(a, a);
+    const double xd = (double)x;
+    const double y = __builtin_amdgcn_rsq(xd);
+    const double h = 0.5 * y;
+    double g = xd * y;
+    g = __builtin_fma(__builtin_fma(-g, g, xd), h, g);
+    g = __builtin_fma(__builtin_fma(-g, g, xd), h, g);
+    const float l = (float)g;
+    const bool special = __builtin_isfpclass(x, kZeroOrInf);
+    len = special ? x : l;
+    return mul_recip(a, special ? y : refine(y, __builtin_fma(-(double)l, y, 1.0)));
+}
+__device__ __forceinline__ f3 normalize(f3 a)
+{
+    float len;
+    return normalize_len(a, len);
+}
 __device__ __forceinline__ float gmax(float a, float b) { return fmaxf(a, b); }
 __device__ __forceinline__ float gmin(float a, float b) { return fminf(a, b); }
 __device__ __forceinline__ float gclamp(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
@@ -186,24 +241,88 @@ __device__ __forceinline__ double exp_d(double t)  // finite t, |t| < 700
 }
 }  // namespace detail
 
+// cos and sin.  A shorter evaluation settles nearly every argument: its
+// relative error is below a known bound, and where no midpoint of two floats
+// lies within that bound every value in the interval rounds to the same
+// float, so also the longer evaluation's (sincos_d).  The 29 bits that the
+// rounding drops say how far the nearest midpoint is.  A lane in 2^15 (cos) or
+// 2^18 (sin and cos) takes the longer way, as do |x| >= 2^27 and NaN.
+//   cos x = -(-1)^n sin(x - (n + 1/2) pi), n = the nearest integer below: one
+//   odd polynomial on [-pi/2, pi/2] (relative error 2^-41.7), no quadrants.
+//   362 -> 144 cycles of a SIMD; sin and cos of one angle 386 -> 188.
+// The polynomials interpolate (sin r - r) / r^3 and (cos r - 1 + r^2/2) / r^4
+// at the Chebyshev nodes of r^2's interval.
+namespace detail {
+// The float nearest y; ok when nothing within `ulps` ulps of y rounds elsewhere.
+__device__ __forceinline__ float round_sure(double y, uint32_t ulps, bool& ok)
+{
+    const uint32_t low = (uint32_t)__double2loint(y) & 0x1FFFFFFFu;
+    ok = low - (0x10000000u - ulps) > 2u * ulps;
+    return (float)y;
+}
+// Out of line: rarely reached, and inlined at every call of rand() it takes
+// the registers of the common way.
+__device__ __attribute__((noinline)) float2 sincos_long(float x)
+{
+    double s, c;
+    sincos_d((double)x, s, c);
+    return make_float2((float)s, (float)c);
+}
+}  // namespace detail
 __device__ __forceinline__ float cos_f(float x)
 {
-    double s, c;
-    detail::sincos_d((double)x, s, c);
-    return (float)c;
-}
-__device__ __forceinline__ float sin_f(float x)
-{
-    double s, c;
-    detail::sincos_d((double)x, s, c);
-    return (float)s;
+    const double xd = (double)x;
+    const double n = rint(__builtin_fma(xd, kd(0.3183098861837907), -0.5));
+    const double m = n + 0.5;
+    double r = __builtin_fma(-m, kd(2.0 * detail::kPio2_1), xd);
+    r = __builtin_fma(-m, kd(2.0 * detail::kPio2_2), r);
+    const double z = r * r;
+    double p = __builtin_fma(z, kd(1.550181221369837e-10), kd(-2.5036706289295077e-08));
+    p = __builtin_fma(z, p, kd(2.7557122430609883e-06));
+    p = __builtin_fma(z, p, kd(-0.0001984126870331528));
+    p = __builtin_fma(z, p, kd(0.008333333330925171));
+    p = __builtin_fma(z, p, kd(-0.16666666666658406));
+    bool ok;
+    float y = detail::round_sure(__builtin_fma(r * z, p, r), 1u << 13, ok);   // 2^-40
+    y = __uint_as_float(__float_as_uint(y) ^ (~((uint32_t)(int)n) << 31));
+    if (__builtin_expect(!(ok && fabsf(x) < 0x1p27f), 0)) y = detail::sincos_long(x).y;
+    return y;
 }
 __device__ __forceinline__ void sincos_f(float x, float& s, float& c)
 {
-    double sd, cd;
-    detail::sincos_d((double)x, sd, cd);
-    s = (float)sd;
-    c = (float)cd;
+    const double xd = (double)x;
+    const double n = rint(xd * kd(detail::kTwoOverPi));
+    double r = __builtin_fma(-n, kd(detail::kPio2_1), xd);
+    r = __builtin_fma(-n, kd(detail::kPio2_2), r);
+    const double z = r * r;
+    double p = __builtin_fma(z, kd(-2.4805011207486557e-08), kd(2.7555984173088083e-06));   // 2^-45.7
+    p = __builtin_fma(z, p, kd(-0.00019841266894627223));
+    p = __builtin_fma(z, p, kd(0.008333333331056203));
+    p = __builtin_fma(z, p, kd(-0.1666666666666385));
+    double q = __builtin_fma(z, kd(2.070015349613916e-09), kd(-2.7556364863807e-07));       // 2^-50
+    q = __builtin_fma(z, q, kd(2.4801585195001366e-05));
+    q = __builtin_fma(z, q, kd(-0.0013888888887260882));
+    q = __builtin_fma(z, q, kd(0.04166666666666465));
+    q = __builtin_fma(z, q, -0.5);
+    bool oks, okc;
+    const float fs = detail::round_sure(__builtin_fma(r * z, p, r), 1u << 10, oks);  // 2^-43
+    const float fc = detail::round_sure(__builtin_fma(z, q, 1.0), 1u << 10, okc);
+    // Quadrant n: (s, c) = (fs, fc), (fc, -fs), (-fs, -fc), (-fc, fs).
+    const uint32_t k = (uint32_t)(int)n;
+    const bool odd = (k & 1u) != 0u;
+    s = __uint_as_float(__float_as_uint(odd ? fc : fs) ^ ((k << 30) & 0x80000000u));
+    c = __uint_as_float(__float_as_uint(odd ? fs : fc) ^ (((k + 1u) << 30) & 0x80000000u));
+    if (__builtin_expect(!(oks && okc && fabsf(x) < 0x1p27f), 0)) {
+        const float2 sc = detail::sincos_long(x);
+        s = sc.x;
+        c = sc.y;
+    }
+}
+__device__ __forceinline__ float sin_f(float x)
+{
+    float s, c;
+    sincos_f(x, s, c);
+    return s;
 }
 __device__ __forceinline__ float pow5(float x)
 {
@@ -237,6 +356,8 @@ constexpr float kTwoPi = 6.28318530718f;       // 2.0 * PI
 constexpr float kInvGamma = 0.45454545454545453f; // 1.0 / 2.2 (:588)
 constexpr float kAttSub = 0.001f;              // :478
 constexpr float kAttDiv = 0.999f;              // 1 - 0.001 (:478)
+constexpr double kAttDivR = 1.0 / (double)kAttDiv;   // for mul_recip
+constexpr double kPiR = 1.0 / (double)kPi;
 constexpr float kK1x = 23.14069263277926f;     // :229
 constexpr float kK1y = 2.665144142690225f;     // :230
 constexpr float kHashScale = 12345.6789f;      // :233
@@ -253,14 +374,18 @@ __device__ __forceinline__ float rng_next(float& salt, float cx, float cy)
 }
 
 // jitter, Assets/Tracer.comp:256-263.
-__device__ __forceinline__ f3 jitter(f3 d, float phi, float sina, float cosa)
+// w = normalize(d).
+__device__ __forceinline__ f3 jitter_w(f3 w, float phi, float sina, float cosa)
 {
-    const f3 w = normalize(d);
     const f3 u = normalize(cross(f3{w.y, w.z, w.x}, w));
     const f3 v = cross(w, u);
     float sp, cp;
     sincos_f(phi, sp, cp);
     return add(muls(add(muls(u, cp), muls(v, sp)), sina), muls(w, cosa));
+}
+__device__ __forceinline__ f3 jitter(f3 d, float phi, float sina, float cosa)
+{
+    return jitter_w(normalize(d), phi, sina, cosa);
 }
 
 // Assets/Tracer.comp:265-312.

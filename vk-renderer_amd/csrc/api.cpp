@@ -83,6 +83,43 @@ bool device_build(vkr_ctx* ctx, Scene* sc, uint32_t n, BuildInput bi, uint32_t d
     return true;
 }
 
+// The records of a scene that is traced by scanning (scan.hpp): few
+// primitives, and coordinates below 2^40, so that no term of a sphere test
+// comes near overflow and powers of two can be taken out of it.
+struct ScanPlan {
+    bool ok = false;
+    float r_max = 0.0f;
+    std::vector<float4> sph;
+    std::vector<TriRecord> tris;
+};
+
+ScanPlan scan_plan(const vkr_scene_desc& d)
+{
+    ScanPlan p;
+    if (scan_units(d.n_spheres, d.n_tris) > kScanUnitsPool) return p;
+    for (uint32_t i = 0; i < d.n_spheres; ++i) {
+        const vkr_sphere& s = d.spheres[i];
+        for (int k = 0; k < 3; ++k)
+            if (!(std::fabs(s.P[k]) < 0x1p40f)) return p;
+        if (!(std::fabs(s.r) < 0x1p40f)) return p;
+        p.r_max = std::max(p.r_max, std::fabs(s.r));
+        p.sph.push_back(make_float4(s.P[0], s.P[1], s.P[2], s.r * s.r));
+    }
+    for (uint32_t i = 0; i < d.n_tris; ++i) {
+        const vkr_triangle& t = d.tris[i];
+        TriRecord r{};
+        for (int k = 0; k < 3; ++k) {
+            r.v0[k] = t.v0[k];
+            r.e1[k] = t.v1[k] - t.v0[k];
+            r.e2[k] = t.v2[k] - t.v0[k];
+        }
+        r.key = i;
+        p.tris.push_back(r);
+    }
+    p.ok = true;
+    return p;
+}
+
 }  // namespace
 }  // namespace vkr
 
@@ -236,6 +273,12 @@ vkr_error vkr_scene_upload(vkr_ctx* ctx, const vkr_scene_desc* desc, uint32_t* o
     VKR_HIP(sc->emitters.alloc(std::max<size_t>(desc->n_spheres, 1u) * sizeof(uint32_t)));
     if (!em.empty()) VKR_HIP(hipMemcpy(sc->emitters.p, em.data(), em.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
 
+    const ScanPlan scan = scan_plan(*desc);
+    if (scan.ok) {
+        VKR_HIP(sc->scan_sph.upload(scan.sph.data(), scan.sph.size() * sizeof(float4)));
+        VKR_HIP(sc->scan_tris.upload(scan.tris.data(), scan.tris.size() * sizeof(TriRecord)));
+    }
+
     DevScene& d = sc->dev;
     d.nodes = sc->nodes.as<BvhNode>();
     d.tris = sc->tris.as<TriRecord>();
@@ -258,6 +301,10 @@ vkr_error vkr_scene_upload(vkr_ctx* ctx, const vkr_scene_desc* desc, uint32_t* o
     d.stack_needed = stack;
     for (int k = 0; k < 3; ++k) d.sph_c[k] = bo.sph_c[k];
     d.sph_r = bo.sph_r;
+    d.scan = scan.ok ? 1u : 0u;
+    d.scan_reach = bo.sph_r + scan.r_max;
+    d.scan_sph = sc->scan_sph.as<float4>();
+    d.scan_tris = sc->scan_tris.as<TriRecord>();
 
     sc->serial = ctx->next_serial++;
     vkr_scene_info& in = sc->info;
@@ -454,7 +501,8 @@ vkr_error vkr_trace_frame(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd
         a.chunk = chunk ? chunk : kDefaultChunk;
         PathVariant v{block, stack, (ctx->flags & VKR_CTX_COUNT_WORK) != 0, false,
                       use_ray_pool(params->flags, s->dev.n_emitters)};
-        if (!tuned) {
+        v.scan = !v.count && use_scan(s->dev, v.pool);
+        if (!tuned && !v.scan) {
             v.stack = default_stack(v, a.total, s->info.depth, ctx->device);
             // The 64-entry-stack kernel runs best in one-wave workgroups
             // (512^2 with 64 spheres: 0.52 against 0.61 ms at 128 lanes).
@@ -538,7 +586,8 @@ vkr_error vkr_trace_frame_static(vkr_ctx* ctx, uint32_t scene, const vkr_frame_d
         a.chunk = chunk ? chunk : kDefaultChunk;
         PathVariant v{block, stack, (ctx->flags & VKR_CTX_COUNT_WORK) != 0, false,
                       use_ray_pool(params->flags, s->dev.n_emitters)};
-        if (!tuned) {
+        v.scan = !v.count && use_scan(s->dev, v.pool);
+        if (!tuned && !v.scan) {
             v.stack = default_stack(v, a.total, s->info.depth, ctx->device);
             // The static records cap the pooled grid below what even 4 waves
             // keep resident; then the fifth wave cannot help.

@@ -27,6 +27,7 @@ struct BatchPlan {
     uint32_t tree_depth = 0;      // the deepest of the jobs' trees
     uint64_t total = 0;
     bool pool = false;            // some job wants the pooled kernel
+    bool scan = true;             // every job's scene is scanned (scan.hpp)
 };
 
 vkr_error plan_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, BatchPlan& plan)
@@ -57,6 +58,7 @@ vkr_error plan_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, BatchP
     }
     plan.start[n] = (uint32_t)off;
     plan.total = off;
+    for (const JobDesc& j : plan.jobs) plan.scan = plan.scan && use_scan(j.sc, plan.pool);
     return VKR_SUCCESS;
 }
 
@@ -79,7 +81,7 @@ PathLaunch batch_launch(const BatchPlan& plan, const JobDesc* djobs, const uint3
 // kernel on the job table: its job is uniform over the grid.
 PathVariant batch_variant(const BatchPlan& plan, uint32_t block, bool count)
 {
-    return PathVariant{block, plan.stack, count, plan.jobs.size() > 1u, plan.pool};
+    return PathVariant{block, plan.stack, count, plan.jobs.size() > 1u, plan.pool, plan.scan && !count};
 }
 
 uint32_t batch_grid(const BatchPlan& plan, const PathVariant& v, int device)

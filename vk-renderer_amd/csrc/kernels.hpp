@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <stddef.h>
 #include <stdint.h>
 
@@ -28,7 +29,32 @@ struct DevScene {
     uint32_t n_materials, flags, has_bvh, stack_needed;
     uint32_t emitters_bounded;      // every emitter: |emissive| < 2^20, 2^-20 <= r <= 2^20
     float sph_c[3], sph_r;          // every sphere centre lies within sph_r of sph_c
+    // Scenes of a few primitives, traced by scanning (scan.hpp, use_scan).
+    uint32_t scan;                  // 1: the scan records exist
+    float scan_reach;               // sph_r + the largest radius
+    const float4* scan_sph;         // scan order: centre, r * r
+    const TriRecord* scan_tris;     // scan order
 };
+
+// A scene is scanned rather than traversed when its tests cost less than the
+// rounds of a tree: by spheres + 2 * triangles (a triangle's test is about two
+// spheres' work).  4 bounces, 2 spp, tree against scan on one MI355X:
+//   single rays (one emitter), 1280x720: 5 spheres 257 / 239 us, 33: 320 / 299,
+//   49: 359 / 354, 65: 372 / 390, 101: 400 / 485;
+//   ray pool (about a quarter emit), 1280x720: 25 spheres 766 / 637 us, 65:
+//   1934 / 1754, 101: 3188 / 3014, 161: 5490 / 6450, but 512x512: 101: 1651 /
+//   1859;
+//   7 spheres and 16 triangles 350 / 306 us, 30 triangles 374 / 344.
+constexpr uint32_t kScanUnits = 56u;       // single rays
+constexpr uint32_t kScanUnitsPool = 80u;   // ray pool
+inline uint32_t scan_units(uint32_t spheres, uint32_t tris)
+{
+    return (uint32_t)std::min<uint64_t>((uint64_t)spheres + 2ull * tris, 0xFFFFFFFFull);
+}
+inline bool use_scan(const DevScene& sc, bool pool)
+{
+    return sc.scan != 0u && scan_units(sc.n_spheres, sc.n_tris) <= (pool ? kScanUnitsPool : kScanUnits);
+}
 
 // One frame of work (a single trace call, or one job of a batch).
 struct JobDesc {
@@ -156,6 +182,7 @@ struct AdjointLaunch {
 struct PathVariant {
     uint32_t block, stack;
     bool count, batch, pool;
+    bool scan = false;   // every job's scene is scanned: no tree, no stack (stack is ignored)
 };
 
 hipError_t launch_path(const PathLaunch& a, const PathVariant& v, uint32_t grid, hipStream_t s);

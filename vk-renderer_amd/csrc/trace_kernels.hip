@@ -25,6 +25,7 @@
 #include <mutex>
 
 #include "kernels.hpp"
+#include "scan.hpp"
 #include "traverse.hpp"
 #include "vkr_device.hpp"
 
@@ -170,6 +171,29 @@ __device__ __forceinline__ const JobDesc& uniform_job(unsigned long long at)
     return *(const JobDesc*)reinterpret_cast<const __attribute__((address_space(4))) JobDesc*>(at);
 }
 
+// Runs body(job) with a job that is the same for all running lanes: once for a
+// launch of one job, else once for each job that the wave's lanes hold (one,
+// but for the few waves at a job's edge).
+template <bool BATCH, class Body>
+__device__ __forceinline__ void for_each_job(const PathLaunch& A, unsigned long long job_at, uint32_t job, bool active,
+                                             Body&& body)
+{
+    if constexpr (!BATCH) {
+        body(uniform_job(job_at));
+    } else {
+        unsigned long long todo = __ballot(active);
+        while (todo) {
+            const uint32_t j = (uint32_t)__builtin_amdgcn_readlane((int)job, __builtin_ctzll(todo));
+            const bool mine = active && job == j;
+            todo &= ~__ballot(mine);
+            const unsigned long long at = (unsigned long long)(A.jobs + j);
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
+            if (mine) body(uniform_job(((unsigned long long)hi << 32) | lo));
+        }
+    }
+}
+
 // The path program of Assets/Tracer.comp:433-593 as a per-lane state machine.
 // Each loop iteration takes every lane one vertex further:
 //   (1) refill idle lanes (their first ray is the primary one);
@@ -193,13 +217,14 @@ __device__ __forceinline__ const JobDesc& uniform_job(unsigned long long at)
 template <int BLOCK, int STACK, bool COUNT, bool BATCH, bool POOL>
 __device__ __forceinline__ void path_program(const PathLaunch& A)
 {
-    __shared__ uint32_t s_stack[STACK * BLOCK];
+    constexpr bool SCAN = STACK == 0;                // no tree: the scene is scanned
+    __shared__ uint32_t s_stack[SCAN ? 1 : STACK * BLOCK];
     __shared__ uint32_t s_occ[BLOCK];                // per lane: occluded shadow rays (bit per slot)
     __shared__ uint2 s_res[BLOCK];                   // per lane: closest hit (prim, t)
     __shared__ uint32_t s_msk[BLOCK];                // per lane: slots holding a ray to trace
     __shared__ uint32_t s_cpre[BLOCK / 64 * kRaySlots];            // per wave and slot: items in lower slots
     __shared__ unsigned long long s_colm[BLOCK / 64 * kRaySlots];  // per wave and slot: lanes holding one
-    uint32_t* stk = s_stack + threadIdx.x;
+    uint32_t* stk = s_stack + (SCAN ? 0u : threadIdx.x);
     const uint32_t wbase = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
     const uint32_t wslot = (wbase >> 6) * kRaySlots;
     char* const wrec = A.lanes + ((size_t)blockIdx.x * (BLOCK / 64) + (wbase >> 6)) * kWaveBytes;
@@ -402,9 +427,15 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
         TravOut tr{kMiss, 0.0f, false};
         if constexpr (!POOL) {
             // (3) At most a shadow ray and a segment per lane, from registers.
-            bool occluded;
-            const JobDesc& jt = BATCH ? A.jobs[job] : uniform_job(job_at);
-            tr = traverse_pair<BLOCK, COUNT>(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, stk, wc, occluded);
+            bool occluded = false;
+            if constexpr (SCAN) {
+                for_each_job<BATCH>(A, job_at, job, has, [&](const JobDesc& jt) __attribute__((always_inline)) {
+                    tr = scan_pair(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, occluded);
+                });
+            } else {
+                const JobDesc& jt = BATCH ? A.jobs[job] : uniform_job(job_at);
+                tr = traverse_pair<BLOCK, COUNT>(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, stk, wc, occluded);
+            }
             if (sh && !occluded) e = add(e, c0);                     // :473, :502
         } else {
             // Path state that the wave's evaluation and tracing do not need
@@ -474,8 +505,35 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            traverse_pool<BLOCK, COUNT, BATCH>(BATCH ? A.jobs : &uniform_job(job_at), nrays, s_cpre + wslot, s_colm + wslot,
-                                               s_occ + wbase, s_res + wbase, wrec, stk, wc);
+            if constexpr (SCAN) {
+                for (uint32_t base = 0; base < nrays; base += 64u) {
+                    const uint32_t i = base + __lane_id();
+                    const bool act = i < nrays;
+                    uint32_t k = 0, lo = 0, rj = 0;
+                    f3 o{}, d{};
+                    float tm = 0.0f;
+                    if (act) {
+                        pool_item(s_cpre + wslot, s_colm + wslot, i, k, lo);
+                        const float4 h = *reinterpret_cast<const float4*>(wrec + (kWHead + lo * 16u));
+                        const float4 r = *reinterpret_cast<const float4*>(wrec + (kWSlotD + (k * 64u + lo) * 16u));
+                        o = f3{h.x, h.y, h.z};
+                        rj = __float_as_uint(h.w);
+                        d = f3{r.x, r.y, r.z};
+                        tm = r.w;
+                    }
+                    TravOut t{kMiss, 0.0f, false};
+                    for_each_job<BATCH>(A, job_at, rj, act, [&](const JobDesc& jt) __attribute__((always_inline)) {
+                        t = scan_ray(jt.sc, o, d, tm, jt.eps, k != 0u, act);
+                    });
+                    if (act) {
+                        if (k == 0u) s_res[wbase + lo] = make_uint2(t.prim, __float_as_uint(t.t));
+                        else if (t.hit) atomicOr(s_occ + wbase + lo, 1u << k);
+                    }
+                }
+            } else {
+                traverse_pool<BLOCK, COUNT, BATCH>(BATCH ? A.jobs : &uniform_job(job_at), nrays, s_cpre + wslot, s_colm + wslot,
+                                                   s_occ + wbase, s_res + wbase, wrec, stk, wc);
+            }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -730,7 +788,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
 // SIMD (its spills are all in per-step code, outside the pool's traversal
 // loops); with deeper stacks LDS allows 4 waves (128 VGPRs).
 template <int BLOCK, int STACK, bool BATCH, bool POOL>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(STACK <= 24 ? 5 : 4))) void k_path(const PathLaunch A)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(STACK == 0 ? 4 : STACK <= 24 ? 5 : 4))) void k_path(const PathLaunch A)
 {
     path_program<BLOCK, STACK, false, BATCH, POOL>(A);
 }
@@ -1020,8 +1078,16 @@ const void* fn_flags(const PathVariant& v)
     return v.batch ? fn_pool<BLOCK, STACK, false, true>(v.pool) : fn_pool<BLOCK, STACK, false, false>(v.pool);
 }
 
+// The scanning kernels have no stack and no counting variant.
+template <int BLOCK>
+const void* fn_scan(const PathVariant& v)
+{
+    return v.batch ? fn_pool<BLOCK, 0, false, true>(v.pool) : fn_pool<BLOCK, 0, false, false>(v.pool);
+}
+
 const void* kernel_ptr(const PathVariant& v)
 {
+    if (v.scan) return v.block == 64 ? fn_scan<64>(v) : v.block == 128 ? fn_scan<128>(v) : fn_scan<256>(v);
     if (v.block == 64) return v.stack <= 24 ? fn_flags<64, 24>(v) : v.stack <= 32 ? fn_flags<64, 32>(v) : fn_flags<64, 64>(v);
     if (v.block == 128) return v.stack <= 24 ? fn_flags<128, 24>(v) : v.stack <= 32 ? fn_flags<128, 32>(v) : fn_flags<128, 64>(v);
     return v.stack <= 24 ? fn_flags<256, 24>(v) : v.stack <= 32 ? fn_flags<256, 32>(v) : fn_flags<256, 64>(v);
@@ -1051,7 +1117,7 @@ uint32_t persistent_grid(const PathVariant& v, int device)
     for (int i = 0; i < n; ++i) {
         const Entry& c = cache[i];
         if (c.device == device && c.v.block == v.block && c.v.stack == v.stack && c.v.count == v.count &&
-            c.v.batch == v.batch && c.v.pool == v.pool)
+            c.v.batch == v.batch && c.v.pool == v.pool && c.v.scan == v.scan)
             return c.grid;
     }
     int per_cu = 0;

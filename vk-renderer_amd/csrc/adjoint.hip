@@ -66,9 +66,9 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(const AdjointLaunch A)
     }
 
     bool has = false;
-    const uint32_t lanes = gridDim.x * BLOCK;
     ItemPool pool;
-    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
+               gridDim.x * (BLOCK / 64), 64u);
     float uvx = 0.0f, uvy = 0.0f, salt = 0.0f, salt0 = 0.0f;
     uint32_t smp = 0, depth = 0, phase = kPhTrace, pass = MODE, zb = 0, nchain = 0, cstar = 0, hs = kMiss;
     uint32_t pix = 0;
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(const AdjointLaunch A)
     };
 
     while (true) {
-        pool.refill(cursor, A.total, lanes, 32u, has, claim);
+        pool.refill(cursor, A.total, 32u, has, claim);
         if (__ballot(has) == 0) {
             if (pool.dry) break;
             continue;

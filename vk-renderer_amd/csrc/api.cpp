@@ -416,23 +416,23 @@ static vkr_error ensure_adj_samples(vkr_ctx* ctx, size_t n)
 // Trees of depth <= 23 can take the 24-entry-stack kernel, which keeps 5
 // waves per SIMD resident (4 with the 32-entry stack, 2 to 3 with the
 // 64-entry one, both with more registers and fewer spills).  Untuned
-// launches choose by the image size against the lanes the 4-wave kernel
-// keeps resident, and by the tree's depth (autotuner tables, one MI355X):
-// - trees deeper than 8 levels, where node fetches dominate: the fifth wave
-//   pays off only with well over twice those pixels (1080p soup frame: 89
-//   against 95 ms; a 512 x 512 soup frame 1% slower), else the 32-entry
-//   kernel;
-// - shallow trees, where shading dominates: the 32-entry kernel (1024^2
-//   reference scene: 2.02 against 2.15 ms, 2048^2: 7.0 against 7.6 ms), or
-//   the 64-entry one when the grid holds every pixel at once (512^2 with 64
-//   spheres: 0.61 against 0.66 ms; 256^2 adjoint scene: 1.43 against
-//   1.48 ms).
+// launches choose by the tree's depth and, with single rays, by the image
+// size against the lanes the 4-wave kernel keeps resident (one MI355X):
+// - trees deeper than 8 levels, where node fetches dominate: the pooled
+//   kernel takes the fifth wave at any size, as narrow waves fill the grid
+//   (256^2 frame of a 50k-triangle soup 7.4 against 8.6 ms); with single rays
+//   it pays off only with well over twice the resident pixels;
+// - shallow trees, where shading dominates: the 32-entry kernel (160 spheres,
+//   a quarter lights, 256^2: 0.74 against 0.78 ms with 24 entries, 0.85 with
+//   64), or for single rays the 64-entry one when the grid holds every pixel
+//   at once.
 static uint32_t default_stack(const PathVariant& v, uint32_t total, uint32_t depth, int device)
 {
     if (v.stack != 24u) return v.stack;
     PathVariant v4 = v;
     v4.stack = 32u;
     const uint64_t resident4 = (uint64_t)persistent_grid(v4, device) * v.block;
+    if (v.pool) return depth <= 8u ? 32u : 24u;
     if (depth <= 8u) return (uint64_t)total <= resident4 ? 64u : 32u;
     return (uint64_t)total > 2u * resident4 ? 24u : 32u;
 }
@@ -511,8 +511,9 @@ vkr_error vkr_trace_frame(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd
         // Persistent: one resident grid.  One pixel per lane: launches of at
         // most kMaxPlainLanes lanes each, in pool order.
         const uint32_t step = persistent ? a.total : kMaxPlainLanes;
-        const uint32_t grid = persistent ? std::min(persistent_grid(v, ctx->device), (a.total + block - 1u) / block)
-                                         : (std::min(a.total, step) + block - 1u) / block;
+        uint32_t grid = (std::min(a.total, step) + block - 1u) / block;
+        a.width = 64u;
+        if (persistent) persistent_shape(v, a.total, s->dev.n_emitters, ~0u, ctx->device, grid, a.width);
         if (v.pool) {
             const vkr_error le = ensure_lanes(ctx, (size_t)grid * block);
             if (le != VKR_SUCCESS) return le;
@@ -597,19 +598,19 @@ vkr_error vkr_trace_frame_static(vkr_ctx* ctx, uint32_t scene, const vkr_frame_d
                 v.stack = 32u;
         }
         const uint32_t step = persistent ? a.total : kMaxPlainLanes;
-        uint32_t grid = persistent ? std::min(persistent_grid(v, ctx->device), (a.total + block - 1u) / block)
-                                   : (std::min(a.total, step) + block - 1u) / block;
+        uint32_t grid = (std::min(a.total, step) + block - 1u) / block;
+        a.width = 64u;
+        // The ray records of every resident lane must fit the array: a
+        // persistent grid is capped to them, a one-pixel-per-lane launch
+        // (one record per pixel) is refused when they do not.
+        const uint32_t cap = v.pool ? (uint32_t)(max_lanes / block) : ~0u;
+        if (cap == 0) return fail(VKR_INVALID_ARGUMENT, "workgroup too large for the static scratch");
+        if (!persistent && grid > cap)
+            return fail(VKR_INVALID_ARGUMENT,
+                        "VKR_SCHED_PLAIN with the ray pool needs one ray record per pixel, more than the static "
+                        "scratch holds (VKR_STATIC_SCRATCH_LANE_BYTES); use the persistent schedule");
+        if (persistent) persistent_shape(v, a.total, s->dev.n_emitters, cap, ctx->device, grid, a.width);
         if (v.pool) {
-            // The ray records of every resident lane must fit the array: a
-            // persistent grid is capped to them, a one-pixel-per-lane launch
-            // (one record per pixel) is refused when they do not.
-            const uint32_t cap = (uint32_t)(max_lanes / block);
-            if (!persistent && (size_t)grid * block > max_lanes)
-                return fail(VKR_INVALID_ARGUMENT,
-                            "VKR_SCHED_PLAIN with the ray pool needs one ray record per pixel, more than the static "
-                            "scratch holds (VKR_STATIC_SCRATCH_LANE_BYTES); use the persistent schedule");
-            if (cap == 0) return fail(VKR_INVALID_ARGUMENT, "workgroup too large for the static scratch");
-            grid = std::min(grid, cap);
             a.lanes = lanes;
         }
         VKR_HIP(launch_zero_counters(cnt, pool, st));

@@ -27,6 +27,7 @@ struct BatchPlan {
     uint32_t tree_depth = 0;      // the deepest of the jobs' trees
     uint64_t total = 0;
     bool pool = false;            // some job wants the pooled kernel
+    uint32_t emitters = ~0u;      // the fewest of any job
     bool scan = true;             // every job's scene is scanned (scan.hpp)
 };
 
@@ -51,6 +52,7 @@ vkr_error plan_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, BatchP
         plan.jobs[i] = make_job(*s, jb.frame_data, jb.params, &jb.outputs);
         plan.stack = std::max(plan.stack, s->dev.stack_needed);
         plan.tree_depth = std::max(plan.tree_depth, s->info.depth);
+        plan.emitters = std::min(plan.emitters, s->dev.n_emitters);
         plan.pool = plan.pool || use_ray_pool(jb.params.flags, s->dev.n_emitters);
         plan.start[i] = (uint32_t)off;
         off += (uint64_t)plan.jobs[i].n_tiles * 64u;
@@ -82,12 +84,6 @@ PathLaunch batch_launch(const BatchPlan& plan, const JobDesc* djobs, const uint3
 PathVariant batch_variant(const BatchPlan& plan, uint32_t block, bool count)
 {
     return PathVariant{block, plan.stack, count, plan.jobs.size() > 1u, plan.pool, plan.scan && !count};
-}
-
-uint32_t batch_grid(const BatchPlan& plan, const PathVariant& v, int device)
-{
-    const uint32_t need = (uint32_t)((plan.total + v.block - 1u) / v.block);
-    return std::max(1u, std::min(persistent_grid(v, device), need));
 }
 
 bool valid_block(uint32_t b) { return b == 0 || b == 64 || b == 128 || b == 256; }
@@ -134,9 +130,9 @@ struct BatchShape {
 // autotuner's choice for this job set (which may also raise the stack
 // depth), else 128 lanes and the default chunk.  Untuned batches whose trees
 // all have at most 8 levels take the register-rich kernels, as single frames
-// do (they shade more than they fetch nodes): the 64-entry-stack kernel when
-// the grid of the 4-wave one holds every pool entry at once, else the
-// 32-entry one.
+// do (they shade more than they fetch nodes): the 32-entry kernel, or with
+// single rays the 64-entry one when the grid of the 4-wave one holds every
+// pool entry at once.
 BatchShape batch_shape(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, BatchPlan& plan, uint32_t block,
                        uint32_t chunk)
 {
@@ -158,7 +154,7 @@ BatchShape batch_shape(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, Batc
     if (!tuned && plan.stack == 24u && plan.tree_depth <= 8u) {
         const PathVariant v4{s.block, 32u, false, plan.jobs.size() > 1u, plan.pool};
         const uint64_t resident4 = (uint64_t)persistent_grid(v4, ctx->device) * s.block;
-        plan.stack = plan.total <= resident4 ? 64u : 32u;
+        plan.stack = !plan.pool && plan.total <= resident4 ? 64u : 32u;
     }
     return s;
 }
@@ -208,7 +204,8 @@ vkr_error vkr_trace_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n_jo
     PathLaunch a = batch_launch(plan, ctx->jobs.as<JobDesc>(), ctx->job_start.as<uint32_t>(), n_jobs, sh.chunk, pool,
                                 cnt);
     const PathVariant v = batch_variant(plan, sh.block, count);
-    const uint32_t grid = batch_grid(plan, v, ctx->device);
+    uint32_t grid = 0, width = 64u;
+    persistent_shape(v, plan.total, plan.emitters, ~0u, ctx->device, grid, width);
     const vkr_error ce = check_cursor(plan, grid, sh.block);
     if (ce != VKR_SUCCESS) return ce;
     if (v.pool) {
@@ -216,6 +213,7 @@ vkr_error vkr_trace_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n_jo
         if (le != VKR_SUCCESS) return le;
         a.lanes = ctx->lanes.as<char>();
     }
+    a.width = width;
     VKR_HIP(launch_zero_counters(cnt, pool, st));
     VKR_HIP(hipEventRecord(ctx->ev0, st));
     VKR_HIP(launch_path(a, v, grid, st));
@@ -238,7 +236,8 @@ vkr_error vkr_batch_graph_create(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32
     const bool count = (ctx->flags & VKR_CTX_COUNT_WORK) != 0;
     const BatchShape sh = batch_shape(ctx, jobs, n_jobs, plan, block, chunk);
     const PathVariant v = batch_variant(plan, sh.block, count);
-    const uint32_t grid = batch_grid(plan, v, ctx->device);
+    uint32_t grid = 0, width = 64u;
+    persistent_shape(v, plan.total, plan.emitters, ~0u, ctx->device, grid, width);
     const vkr_error ce = check_cursor(plan, grid, sh.block);
     if (ce != VKR_SUCCESS) return ce;
 
@@ -258,6 +257,7 @@ vkr_error vkr_batch_graph_create(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32
         a.lanes = g->lanes.as<char>();
     }
 
+    a.width = width;
     // Capture on a private stream: a fill kernel resets the pool cursor and the
     // counters (no memset nodes), then the persistent batch kernel.
     hipStream_t cap = nullptr;

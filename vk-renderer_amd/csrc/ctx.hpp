@@ -288,6 +288,36 @@ inline bool use_ray_pool(uint32_t flags, uint32_t n_emitters)
     return n_emitters >= 2u;
 }
 
+// Workgroups of a persistent launch over `total` pixels, and how many lanes of
+// each wave take pixels (kernels.hpp: PathLaunch::width).  At most max_grid
+// workgroups (what the ray records hold).
+//
+// A pooled wave needs few pixels to keep its lanes busy: each one queues the
+// rays of up to 31 emitters, which any lane evaluates and traces.  So an image
+// too small to give every SIMD eight rounds of full waves gives each wave
+// fewer pixels and runs more waves, as long as its pixels times the emitters
+// still fill a wave.  A path of a single-ray wave needs a lane of its own, so
+// there narrow waves only pay while SIMDs would stay empty.
+// Width 64 against the chosen one (one MI355X): ray pool, 50k-triangle soup
+// 256^2 21.4 -> 7.4 ms (8 pixels a wave), 512^2 14.4 -> 9.5 (32), 5k-triangle
+// soup 64^2 7.9 -> 1.1 (1); 65 spheres 512^2 484 -> 395 us (32), 256^2 655 ->
+// 345 (8); 4 emitters 256^2 1021 -> 597 (16; 8: 648).  Single rays: 64^2
+// reference scene 102 -> 91 us (4), 64^2 16 spp adjoint scene 566 -> 517 (4),
+// but 256^2 563 -> 600 (32).
+inline void persistent_shape(const PathVariant& v, uint64_t total, uint32_t n_emitters, uint32_t max_grid, int device,
+                             uint32_t& grid, uint32_t& width)
+{
+    const uint32_t waves = v.block / 64u;   // of a workgroup
+    const uint32_t resident = std::min(persistent_grid(v, device), max_grid);
+    const uint32_t simds = 4u * compute_units(device);
+    const uint64_t rounds = v.pool ? std::min<uint64_t>(8u * simds, 2ull * resident * waves) : simds;
+    const uint32_t least = v.pool ? (64u + std::max(n_emitters, 1u) - 1u) / std::max(n_emitters, 1u) : 1u;
+    width = 64u;
+    while (width / 2u >= least && total < rounds * width) width /= 2u;
+    const uint64_t need = (total + (uint64_t)width * waves - 1u) / ((uint64_t)width * waves);
+    grid = (uint32_t)std::max<uint64_t>(1u, std::min<uint64_t>(resident, need));
+}
+
 inline const TuneEntry* find_tuned(const vkr_ctx* ctx, uint32_t scene, const vkr_trace_params& p)
 {
     for (const TuneEntry& t : ctx->tuned)

@@ -156,6 +156,7 @@ struct PathLaunch {
     uint32_t persistent;          // 0: one pixel per lane; 1: refill from pool
     uint32_t base;                // one pixel per lane: pool index of the launch's lane 0
     uint32_t chunk;               // refill when at least this many lanes idle
+    uint32_t width;               // lanes of a wave that take pixels (the others only help with its rays)
     uint32_t* pool;               // persistent pool cursor (device)
     CounterRef counters;
     char* lanes;                  // ray records: one kWaveBytes block per wave of the grid
@@ -196,6 +197,7 @@ hipError_t launch_zero_counters(CounterRef c, uint32_t* pool, hipStream_t s);
 // Writes the per-frame fields of a job in a device job table (camera,
 // aspect, seed, light position), in stream order.
 hipError_t launch_set_frame(JobDesc* job, const vkr_frame_data& fd, hipStream_t s);
+uint32_t compute_units(int device);
 // Occupancy-derived persistent grid size for (block, stack).
 uint32_t persistent_grid(const PathVariant& v, int device);
 

@@ -237,9 +237,8 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
 
     // Lane state.
     bool has = false;
-    const uint32_t lanes = gridDim.x * BLOCK;
     ItemPool pool;
-    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + (wbase >> 6));
+    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + (wbase >> 6), gridDim.x * (BLOCK / 64), A.width);
     uint32_t job = 0, px = 0, py = 0;
     float uvx = 0.0f, uvy = 0.0f, salt = 0.0f;
     uint32_t smp = 0, depth = 0;
@@ -338,7 +337,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
     }
 
     while (true) {
-        if (A.persistent) pool.refill(A.pool, A.total, lanes, A.chunk, has, claim);
+        if (A.persistent) pool.refill(A.pool, A.total, A.chunk, has, claim);
         const unsigned long long live = __ballot(has);
         if (live == 0) {
             if (!A.persistent || pool.dry) break;
@@ -1108,6 +1107,16 @@ hipError_t launch_path(const PathLaunch& a, const PathVariant& v, uint32_t grid,
     return hipLaunchKernel(kernel_ptr(v), dim3(grid), dim3(v.block), args, 0, s);
 }
 
+uint32_t compute_units(int device)
+{
+    static thread_local int dev = -1, cus = 0;
+    if (dev != device) {
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 256;
+        dev = device;
+    }
+    return (uint32_t)cus;
+}
+
 uint32_t persistent_grid(const PathVariant& v, int device)
 {
     // Resident workgroups per CU x CUs, cached per (device, variant).
@@ -1124,9 +1133,7 @@ uint32_t persistent_grid(const PathVariant& v, int device)
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_ptr(v), (int)v.block, 0) != hipSuccess ||
         per_cu < 1)
         per_cu = 1;
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1) cus = 256;
-    const uint32_t grid = (uint32_t)(per_cu * cus);
+    const uint32_t grid = (uint32_t)per_cu * compute_units(device);
     if (n < 64) cache[n++] = Entry{device, v, grid};
     return grid;
 }

@@ -507,44 +507,47 @@ __device__ __forceinline__ DevCounters* counter_bank(const CounterRef& c, uint32
     return c.banks + (block & c.mask);
 }
 
-// A wave's view of a launch's pool of work items.  The wave starts with the 64
-// items of its own number; the pool's cursor counts from the grid's lanes up,
-// so the waves of a launch do not open it with a queue of atomics on one
-// address (11.5 ns each).  Later claims take just the idle lanes' items: a
+// A wave's view of a launch's pool of work items, which its lanes 0 .. width - 1
+// take.  The wave starts with the `width` items of its own number; the pool's
+// cursor counts from the last wave's up, so the waves of a launch do not open
+// it with a queue of atomics on one address (11.5 ns each).  Later claims take just the idle lanes' items: a
 // wave that kept a run of items to itself (a share of what is left, up to 64)
 // made fewer claims but left waves idle at the end of the launch while others
 // still held items (1080p heightfield 9.0 -> 11.5 ms, 1024^2 reference scene
 // 2.06 -> 2.50 ms).
 struct ItemPool {
     uint32_t own;             // first of the wave's own items (kNoItem: taken)
+    uint32_t shared;          // items below are the waves' own
+    uint32_t width;           // lanes that take items
     bool dry;                 // nothing is left behind the cursor
     static constexpr uint32_t kNoItem = 0xFFFFFFFFu;
 
-    __device__ __forceinline__ void start(uint32_t wave)
+    __device__ __forceinline__ void start(uint32_t wave, uint32_t waves, uint32_t width_)
     {
-        own = wave * 64u;
+        width = width_;
+        own = wave * width;
+        shared = waves * width;
         dry = false;
     }
     // Gives items to the idle lanes (has == false) once at least `chunk` of
-    // them wait: claim(item) for each.  Every lane of the wave calls it.
+    // them wait, or all: claim(item) for each.  Every lane of the wave calls it.
     template <class Claim>
-    __device__ __forceinline__ void refill(uint32_t* cursor, uint32_t total, uint32_t lanes, uint32_t chunk, bool has,
-                                           Claim&& claim)
+    __device__ __forceinline__ void refill(uint32_t* cursor, uint32_t total, uint32_t chunk, bool has, Claim&& claim)
     {
-        const unsigned long long need = __ballot(!has);
+        const unsigned long long need = __ballot(!has && __lane_id() < width);
         const uint32_t n = (uint32_t)__popcll(need);
-        if (n == 0u || n < chunk || dry) return;
+        if (n == 0u || n < min(chunk, width) || dry) return;
         uint32_t base = own;
         if (own == kNoItem) {
             base = 0u;
             if (__lane_id() == 0) base = atomicAdd(cursor, n);
-            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + lanes;
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base) + shared;
         }
         own = kNoItem;
-        // (Items below `lanes` are the waves' own: a wave whose own items lie
-        // past the total finds the cursor's there too.)
-        dry = base + n >= total && base >= lanes;
-        if (!has) {
+        // (A wave whose own items lie past the total finds the cursor's there
+        // too.)
+        dry = base + n >= total && base >= shared;
+        if ((need >> __lane_id()) & 1ull) {
             const uint32_t g = base + (uint32_t)__popcll(need & ((1ull << __lane_id()) - 1ull));
             if (g < total) claim(g);
         }

@@ -401,15 +401,20 @@ vkr_error vkr_scene_set_sphere_params(vkr_ctx* ctx, uint32_t scene, const float*
     return VKR_SUCCESS;
 }
 
-// Room for the adjoint's first-pass records of n samples in the context.
-// Growing the buffer waits for the device, as for the ray records.
-static vkr_error ensure_adj_samples(vkr_ctx* ctx, size_t n)
+// Points a job at room for the adjoint's first-pass records in the context: one
+// per sample, then one per pixel.  Growing the buffer waits for the device, as
+// for the ray records.
+static vkr_error ensure_adj_records(vkr_ctx* ctx, JobDesc& j)
 {
-    const size_t bytes = n * sizeof(uint2);
-    if (ctx->adj_samples.bytes >= bytes) return VKR_SUCCESS;
-    ctx->adj_key.valid = false;
-    VKR_HIP(hipDeviceSynchronize());
-    VKR_HIP(ctx->adj_samples.alloc(bytes));
+    const size_t pixels = (size_t)j.W * j.H, samples = pixels * j.spp;
+    const size_t bytes = (samples + pixels) * sizeof(uint2);
+    if (ctx->adj_samples.bytes < bytes) {
+        ctx->adj_key.valid = false;
+        VKR_HIP(hipDeviceSynchronize());
+        VKR_HIP(ctx->adj_samples.alloc(bytes));
+    }
+    j.adj_samples = ctx->adj_samples.as<uint2>();
+    j.adj_primary = j.adj_samples + samples;
     return VKR_SUCCESS;
 }
 
@@ -435,6 +440,70 @@ static uint32_t default_stack(const PathVariant& v, uint32_t total, uint32_t dep
     if (v.pool) return depth <= 8u ? 32u : 24u;
     if (depth <= 8u) return (uint64_t)total <= resident4 ? 64u : 32u;
     return (uint64_t)total > 2u * resident4 ? 24u : 32u;
+}
+
+// The path kernel's launches for one frame.
+struct FrameLaunch {
+    PathLaunch a{};
+    PathVariant v{};
+    uint32_t grid = 0, step = 0;
+
+    hipError_t launch(hipStream_t st)
+    {
+        for (uint32_t base = 0; base < a.total; base += step) {
+            a.base = base;
+            const uint32_t g = a.persistent ? grid : (std::min(a.total - base, step) + v.block - 1u) / v.block;
+            const hipError_t e = launch_path(a, v, g, st);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+};
+
+// Plans them: the tuned or default shape, and the context's ray records.
+static vkr_error plan_frame(vkr_ctx* ctx, uint32_t scene, const Scene& s, const vkr_trace_params& params,
+                            const JobDesc& j, bool count, FrameLaunch& f)
+{
+    PathLaunch& a = f.a;
+    a.job = j;
+    a.total = j.n_tiles * 64u;
+    a.pool = ctx->pool.as<uint32_t>();
+    a.counters = banked(ctx->counters);
+    uint32_t block = params.block, chunk = params.chunk, sched = params.sched;
+    uint32_t stack = s.dev.stack_needed;
+    const TuneEntry* tuned = find_tuned(ctx, scene, params);
+    if (const TuneEntry* t = tuned) {
+        if (!block) block = t->block;
+        if (!chunk) chunk = t->chunk;
+        if (sched == VKR_SCHED_AUTO) sched = t->sched;
+        stack = std::max(stack, t->stack);
+    }
+    if (!block) block = 128u;
+    const bool persistent = sched != VKR_SCHED_PLAIN;
+    a.persistent = persistent ? 1u : 0u;
+    a.chunk = chunk ? chunk : kDefaultChunk;
+    PathVariant& v = f.v;
+    v = PathVariant{block, stack, count, false, use_ray_pool(params.flags, s.dev.n_emitters)};
+    v.scan = !v.count && use_scan(s.dev, v.pool);
+    if (!tuned && !v.scan) {
+        v.stack = default_stack(v, a.total, s.info.depth, ctx->device);
+        // The 64-entry-stack kernel runs best in one-wave workgroups
+        // (512^2 with 64 spheres: 0.52 against 0.61 ms at 128 lanes).
+        if (v.stack == 64u && params.block == 0) block = v.block = 64u;
+    }
+    // Persistent: one resident grid.  One pixel per lane: launches of at
+    // most kMaxPlainLanes lanes each, in pool order.
+    f.step = persistent ? a.total : kMaxPlainLanes;
+    uint32_t& grid = f.grid;
+    grid = (std::min(a.total, f.step) + block - 1u) / block;
+    a.width = 64u;
+    if (persistent) persistent_shape(v, a.total, s.dev.n_emitters, ~0u, ctx->device, grid, a.width);
+    if (v.pool) {
+        const vkr_error le = ensure_lanes(ctx, (size_t)grid * block);
+        if (le != VKR_SUCCESS) return le;
+        a.lanes = ctx->lanes.as<char>();
+    }
+    return VKR_SUCCESS;
 }
 
 vkr_error vkr_trace_frame(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd, const vkr_trace_params* params,
@@ -469,9 +538,8 @@ vkr_error vkr_trace_frame(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd
         // The records are rewritten from here on: they describe this frame
         // only once its launch is in the stream.
         ctx->adj_key.valid = false;
-        const vkr_error ae = ensure_adj_samples(ctx, (size_t)j.W * j.H * j.spp);
+        const vkr_error ae = ensure_adj_records(ctx, j);
         if (ae != VKR_SUCCESS) return ae;
-        j.adj_samples = ctx->adj_samples.as<uint2>();
     }
     const CounterRef cnt = banked(ctx->counters);
     uint32_t* pool = ctx->pool.as<uint32_t>();
@@ -481,50 +549,11 @@ vkr_error vkr_trace_frame(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd
         VKR_HIP(launch_whitted(j, cnt, st));
         VKR_HIP(hipEventRecord(ctx->ev1, st));
     } else {
-        PathLaunch a{};
-        a.job = j;
-        a.total = j.n_tiles * 64u;
-        a.pool = pool;
-        a.counters = cnt;
-        uint32_t block = params->block, chunk = params->chunk, sched = params->sched;
-        uint32_t stack = s->dev.stack_needed;
-        const TuneEntry* tuned = find_tuned(ctx, scene, *params);
-        if (const TuneEntry* t = tuned) {
-            if (!block) block = t->block;
-            if (!chunk) chunk = t->chunk;
-            if (sched == VKR_SCHED_AUTO) sched = t->sched;
-            stack = std::max(stack, t->stack);
-        }
-        if (!block) block = 128u;
-        const bool persistent = sched != VKR_SCHED_PLAIN;
-        a.persistent = persistent ? 1u : 0u;
-        a.chunk = chunk ? chunk : kDefaultChunk;
-        PathVariant v{block, stack, (ctx->flags & VKR_CTX_COUNT_WORK) != 0, false,
-                      use_ray_pool(params->flags, s->dev.n_emitters)};
-        v.scan = !v.count && use_scan(s->dev, v.pool);
-        if (!tuned && !v.scan) {
-            v.stack = default_stack(v, a.total, s->info.depth, ctx->device);
-            // The 64-entry-stack kernel runs best in one-wave workgroups
-            // (512^2 with 64 spheres: 0.52 against 0.61 ms at 128 lanes).
-            if (v.stack == 64u && params->block == 0) block = v.block = 64u;
-        }
-        // Persistent: one resident grid.  One pixel per lane: launches of at
-        // most kMaxPlainLanes lanes each, in pool order.
-        const uint32_t step = persistent ? a.total : kMaxPlainLanes;
-        uint32_t grid = (std::min(a.total, step) + block - 1u) / block;
-        a.width = 64u;
-        if (persistent) persistent_shape(v, a.total, s->dev.n_emitters, ~0u, ctx->device, grid, a.width);
-        if (v.pool) {
-            const vkr_error le = ensure_lanes(ctx, (size_t)grid * block);
-            if (le != VKR_SUCCESS) return le;
-            a.lanes = ctx->lanes.as<char>();
-        }
+        FrameLaunch f;
+        const vkr_error fe = plan_frame(ctx, scene, *s, *params, j, (ctx->flags & VKR_CTX_COUNT_WORK) != 0, f);
+        if (fe != VKR_SUCCESS) return fe;
         VKR_HIP(hipEventRecord(ctx->ev0, st));
-        for (uint32_t base = 0; base < a.total; base += step) {
-            a.base = base;
-            const uint32_t g = persistent ? grid : (std::min(a.total - base, step) + block - 1u) / block;
-            VKR_HIP(launch_path(a, v, g, st));
-        }
+        VKR_HIP(f.launch(st));
         VKR_HIP(hipEventRecord(ctx->ev1, st));
         if (rec_adj) ctx->adj_key = adjoint_key(s->serial, *fd, *params);
     }
@@ -739,29 +768,46 @@ vkr_error vkr_adjoint(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd, co
     hipStream_t st = static_cast<hipStream_t>(stream);
     AdjointLaunch a{};
     a.job = make_job(*s, *fd, *params, nullptr);
+    // The second pass hands out one item per (pixel, sample) of whole tiles.
+    if ((uint64_t)a.job.n_tiles * 64u * a.job.spp > kMaxPoolItems)
+        return fail(VKR_UNSUPPORTED, "the adjoint takes at most 0xFF000000 (pixel, sample) pairs per call (8x8 tiles)");
+    // The first pass's records, 8 bytes per (pixel, sample) and 8 per pixel,
+    // are still those of this frame when a recording vkr_trace_frame or an
+    // adjoint wrote them for the same scene version, frame data and trace
+    // parameters.
+    const AdjointKey key = adjoint_key(s->serial, *fd, *params);
+    const bool recorded = same_key(ctx->adj_key, key);
+    if (!recorded) ctx->adj_key.valid = false;
+    const vkr_error ae = ensure_adj_records(ctx, a.job);
+    if (ae != VKR_SUCCESS) return ae;
+    // The first pass is the path kernel without an image.  It needs no ray
+    // pool: where the pool's records cannot be had, it runs without.
+    FrameLaunch f;
+    if (!recorded) {
+        vkr_trace_params p = *params;
+        p.sched = VKR_SCHED_PERSISTENT;
+        p.block = p.chunk = 0;
+        vkr_error fe = plan_frame(ctx, scene, *s, p, a.job, false, f);
+        if (fe == VKR_OUT_OF_MEMORY) {
+            (void)hipGetLastError();
+            p.flags = VKR_TRACE_NO_RAY_POOL;
+            fe = plan_frame(ctx, scene, *s, p, a.job, false, f);
+        }
+        if (fe != VKR_SUCCESS) return fe;
+        f.a.rays_only = 1u;
+    }
     a.d_radiance = d_radiance;
     a.d_params = d_params;
     a.params = s->theta.as<float>();
     a.counters = banked(ctx->counters);
-    a.pool = ctx->pool.as<uint32_t>();
-    a.total = a.job.n_tiles * 64u;
-    // The second pass hands out one item per (pixel, sample) of whole tiles.
-    if ((uint64_t)a.total * a.job.spp > kMaxPoolItems)
-        return fail(VKR_UNSUPPORTED, "the adjoint takes at most 0xFF000000 (pixel, sample) pairs per call (8x8 tiles)");
-    // The first pass's records, 8 bytes per (pixel, sample), are still those
-    // of this frame when a recording vkr_trace_frame or an adjoint wrote
-    // them for the same scene version, frame data and trace parameters.
-    const AdjointKey key = adjoint_key(s->serial, *fd, *params);
-    const bool recorded = same_key(ctx->adj_key, key);
-    if (!recorded) {
-        ctx->adj_key.valid = false;
-        const vkr_error ae = ensure_adj_samples(ctx, (size_t)a.job.W * a.job.H * a.job.spp);
-        if (ae != VKR_SUCCESS) return ae;
-    }
-    a.samples = ctx->adj_samples.as<uint2>();
-    VKR_HIP(launch_zero_counters(a.counters, a.pool, st));
+    a.pool = ctx->pool.as<uint32_t>() + 1;
+    a.total = a.job.n_tiles * 64u * a.job.spp;
+    a.samples = a.job.adj_samples;
+    a.primary = a.job.adj_primary;
+    VKR_HIP(launch_zero_counters(a.counters, ctx->pool.as<uint32_t>(), st));
     VKR_HIP(hipEventRecord(ctx->ev0, st));
-    VKR_HIP(launch_adjoint(a, s->dev.stack_needed, !recorded, st));
+    if (!recorded) VKR_HIP(f.launch(st));
+    VKR_HIP(launch_adjoint(a, s->dev.stack_needed, use_scan(s->dev, false), st));
     VKR_HIP(hipEventRecord(ctx->ev1, st));
     ctx->adj_key = key;
     ctx->timed = true;

@@ -79,6 +79,7 @@ struct JobDesc {
     uint16_t* decisions;
     uint2* adj_samples;           // W*H*spp, pixel-major: (bits of the random-stream position at the
                                   // sample's start, clamp-saturation bits) for the adjoint; NULL: none
+    uint2* adj_primary;           // W*H: (primary hit's primitive, bits of its t) for the adjoint; NULL: none
 };
 
 // Atomics on one address are served one after the other, 11.5 ns each
@@ -154,6 +155,7 @@ struct PathLaunch {
     uint32_t n_jobs;
     uint32_t total;               // pool indices (64 per 8x8 tile)
     uint32_t persistent;          // 0: one pixel per lane; 1: refill from pool
+    uint32_t rays_only;           // count rays, nothing else (the adjoint's first pass)
     uint32_t base;                // one pixel per lane: pool index of the launch's lane 0
     uint32_t chunk;               // refill when at least this many lanes idle
     uint32_t width;               // lanes of a wave that take pixels (the others only help with its rays)
@@ -171,10 +173,11 @@ struct AdjointLaunch {
     float* d_params;              // 7 * n_spheres + 1
     const float* params;          // 7 * n_spheres + 1 (current values)
     CounterRef counters;
-    uint32_t* pool;               // persistent pool cursors: [0] pass 1, [1] pass 2
-    uint32_t total;               // pool indices (64 per 8x8 tile; pass 2: per tile and sample)
-    uint2* samples;               // W*H*spp: (bits of the random-stream position at the sample's
-                                  // start, the pass-1 clamp-saturation bits), pixel-major
+    uint32_t* pool;               // the pool cursor of the second pass
+    uint32_t total;               // pool indices (64 per 8x8 tile and sample)
+    // The first pass's records (JobDesc::adj_samples, adj_primary).
+    const uint2* samples;
+    const uint2* primary;
 };
 
 // One instantiation of the path kernel.  pool: a wave traces up to
@@ -190,8 +193,9 @@ hipError_t launch_path(const PathLaunch& a, const PathVariant& v, uint32_t grid,
 hipError_t launch_whitted(const JobDesc& j, CounterRef c, hipStream_t s);
 hipError_t launch_filter(const uint8_t* cur, const uint8_t* prev, uint32_t sw, uint32_t sh, uint8_t* out,
                          uint32_t dw, uint32_t dh, hipStream_t s);
-// pass1 false: a.samples already holds the first pass's records of this frame.
-hipError_t launch_adjoint(const AdjointLaunch& a, uint32_t stack, bool pass1, hipStream_t s);
+// The adjoint's second pass; a.samples and a.primary hold the first pass's
+// records of this frame.  scan: the scene is scanned (use_scan).
+hipError_t launch_adjoint(const AdjointLaunch& a, uint32_t stack, bool scan, hipStream_t s);
 hipError_t launch_debug(uint32_t op, const float* in, float* out, uint32_t n, hipStream_t s);
 hipError_t launch_zero_counters(CounterRef c, uint32_t* pool, hipStream_t s);
 // Writes the per-frame fields of a job in a device job table (camera,

@@ -395,10 +395,11 @@ __device__ __forceinline__ float schlick(float cosine, float ior)
     r0 = r0 * r0;
     return r0 + (1.0f - r0) * pow5(1.0f - cosine);
 }
+// p = pow5(1 - cos_theta)
+__device__ __forceinline__ f3 fresnel_schlick_p(float p, f3 F0) { return add(F0, muls(ssub(1.0f, F0), p)); }
 __device__ __forceinline__ f3 fresnel_schlick(float cos_theta, f3 F0)
 {
-    const float p = pow5(1.0f - cos_theta);
-    return add(F0, muls(ssub(1.0f, F0), p));
+    return fresnel_schlick_p(pow5(1.0f - cos_theta), F0);
 }
 __device__ __forceinline__ float distribution_ggx(f3 N, f3 H, float roughness)
 {

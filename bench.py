@@ -43,11 +43,11 @@ FP32_PEAK_TFLOPS = 78.6   # non-packed FP32 FMA: 256 CU x 128 FLOP/clk x 2.4 GHz
 # FP32 operations per unit of work (slab test of one box, one Moller-Trumbore
 # triangle test, one sphere test), for the secondary compute figure.
 BOX_FLOP, TRI_FLOP, SPHERE_FLOP = 20, 50, 20
-# Request bytes per unit of work as this build lays them out: a 64-byte node
+# Request bytes per unit of work as this build lays them out: a 48-byte node
 # (two child boxes), a 48-byte triangle record, a 16-byte sphere record plus
 # its 4-byte scan key, a plane's normal and offset, an rgba8 pixel.  The
 # std430 sizes of a Sphere and a Plane are 64 bytes each.
-NODE_B, TRI_B, SPHERE_B, PLANE_B, OUT_B = 64, 48, 20, 16, 4
+NODE_B, TRI_B, SPHERE_B, PLANE_B, OUT_B = 48, 48, 20, 16, 4
 STD430_SPHERE_B = STD430_PLANE_B = 64
 CPU_THREAD_CAP = 16       # a GPU's share of its host's threads
 

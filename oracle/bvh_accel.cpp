@@ -119,41 +119,49 @@ int trace(const void* ap, const float of[3], const float df[3], float eps, int a
         const float ix = inv(d.x), iy = inv(d.y), iz = inv(d.z);
         const float ox = o.x * ix, oy = o.y * iy, oz = o.z * iz;
         const float ax = std::fabs(ix), ay = std::fabs(iy), az = std::fabs(iz);
-        // The sphere subtree's boxes are widened by 2e-3 (|o - C| + R): the
-        // reference's sphere test accepts rays up to ~1e-3 |o - c| outside a
-        // sphere from far away (rounding in its discriminant).
+        // The sphere subtree's boxes are widened by sqrt(r^2 + 64u D^2) - r for
+        // the least radius r and D >= |o - c| for every centre: the
+        // reference's sphere test accepts rays up to that far outside a
+        // sphere (rounding in its discriminant).
         const F3 oc = sub3(o, P3(A.bvh.sph_c));
-        const float pad = 2e-3f * (std::sqrt(dot3(oc, oc)) + A.bvh.sph_r);
-        const float px = std::fmin(pad * ax, 3e38f), py = std::fmin(pad * ay, 3e38f), pz = std::fmin(pad * az, 3e38f);
+        const float D = std::sqrt(dot3(oc, oc)) + A.bvh.sph_r, rmin = A.bvh.sph_rmin;
+        const float q = 0x1p-18f * (D * D);
+        float pad = q / (std::sqrt(std::fma(rmin, rmin, q)) + rmin);
+        pad = pad < 3e38f ? pad : 3e38f;
         float cull = any ? tmax_eps : tmax_eps + win;
         uint32_t stack[128];
         int sp = 0;
         uint32_t ref = 0;
         while (true) {
             if ((int32_t)ref >= 0) {
-                const vkr::BvhNode& n = A.bvh.nodes[ref];
+                const vkr::BvhNode& n = A.bvh.nodes[ref / 3u];
                 ++c_nodes;
                 const float cb = cull + std::fabs(cull) * 1e-5f + 1e-5f;
-                float m;
-                std::memcpy(&m, &n.d[2], 4);
-                const float qx = m * px, qy = m * py, qz = m * pz;
-                auto box = [&](float cx, float ex, float cy, float ey, float cz, float ez, float& nr, float& fr) {
-                    const float a0 = std::fma(cx, ix, -ox), a1 = std::fma(ex, ax, qx);
-                    const float a2 = std::fma(cy, iy, -oy), a3 = std::fma(ey, ay, qy);
-                    const float a4 = std::fma(cz, iz, -oz), a5 = std::fma(ez, az, qz);
-                    nr = std::fmax(std::fmax(a0 - a1, a2 - a3), std::fmax(a4 - a5, 0.0f));
-                    fr = std::fmin(std::fmin(a0 + a1, a2 + a3), std::fmin(a4 + a5, cb));
+                auto half = [](uint16_t h) {   // normal or infinite, never negative
+                    const uint32_t u = (h >> 10) == 31u ? 0x7F800000u : ((uint32_t)h << 13) + (112u << 23);
+                    float f;
+                    std::memcpy(&f, &u, 4);
+                    return f;
+                };
+                auto box = [&](float cx, float cy, float cz, const uint16_t* e, float& nr, float& fr) {
+                    const float ex = std::fma(n.m, pad, half(e[0])), ey = std::fma(n.m, pad, half(e[1]));
+                    const float ez = std::fma(n.m, pad, half(e[2]));
+                    const float a0 = std::fma(cx, ix, -ox), a1 = std::fma(cy, iy, -oy), a2 = std::fma(cz, iz, -oz);
+                    nr = std::fmax(std::fmax(std::fma(-ex, ax, a0), std::fma(-ey, ay, a1)),
+                                   std::fmax(std::fma(-ez, az, a2), 0.0f));
+                    fr = std::fmin(std::fmin(std::fma(ex, ax, a0), std::fma(ey, ay, a1)),
+                                   std::fmin(std::fma(ez, az, a2), cb));
                 };
                 float n0, f0, n1, f1;
-                box(n.a[0], n.a[1], n.a[2], n.a[3], n.b[0], n.b[1], n0, f0);
-                box(n.b[2], n.b[3], n.c[0], n.c[1], n.c[2], n.c[3], n1, f1);
+                box(n.c0[0], n.c0[1], n.c0[2], n.e, n0, f0);
+                box(n.c1x, n.c1yz[0], n.c1yz[1], n.e + 3, n1, f1);
                 const bool h0 = n0 <= f0, h1 = n1 <= f1;
                 if (h0 && h1) {
                     const bool first0 = n0 <= n1;
-                    stack[sp++] = first0 ? n.d[1] : n.d[0];
-                    ref = first0 ? n.d[0] : n.d[1];
+                    stack[sp++] = first0 ? n.ref[1] : n.ref[0];
+                    ref = first0 ? n.ref[0] : n.ref[1];
                 } else if (h0 || h1) {
-                    ref = h0 ? n.d[0] : n.d[1];
+                    ref = h0 ? n.ref[0] : n.ref[1];
                 } else {
                     if (sp == 0) break;
                     ref = stack[--sp];

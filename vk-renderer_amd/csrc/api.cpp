@@ -69,7 +69,7 @@ bool device_build(vkr_ctx* ctx, Scene* sc, uint32_t n, BuildInput bi, uint32_t d
     }
     if (has_sph) {
         offset_inner_refs(sb.nodes, sph_off);
-        const BvhNode top = join_root(root.lo, root.hi, node_off, sph_off);
+        const BvhNode top = join_root(root.lo, root.hi, inner_ref(node_off), inner_ref(sph_off));
         BvhNode* dn = sc->nodes.as<BvhNode>();
         if ((*err = hipMemcpy(dn, &top, sizeof top, hipMemcpyHostToDevice)) != hipSuccess) return false;
         *err = hipMemcpy(dn + sph_off, sb.nodes.data(), sb.nodes.size() * sizeof(BvhNode), hipMemcpyHostToDevice);
@@ -301,6 +301,7 @@ vkr_error vkr_scene_upload(vkr_ctx* ctx, const vkr_scene_desc* desc, uint32_t* o
     d.stack_needed = stack;
     for (int k = 0; k < 3; ++k) d.sph_c[k] = bo.sph_c[k];
     d.sph_r = bo.sph_r;
+    d.sph_rmin = bo.sph_rmin;
     d.scan = scan.ok ? 1u : 0u;
     d.scan_reach = bo.sph_r + scan.r_max;
     d.scan_sph = sc->scan_sph.as<float4>();

@@ -67,45 +67,39 @@ inline void centre_extent(float lo, float hi, float& c, float& e)
     if ((double)e < ed) e = std::nextafter(e, std::numeric_limits<float>::infinity());
 }
 
+inline void put_box(BvhNode& n, int slot, const float* c, const float* e, uint32_t ref)
+{
+    if (slot == 0) {
+        for (int k = 0; k < 3; ++k) n.c0[k] = c[k];
+    } else {
+        n.c1x = c[0];
+        n.c1yz[0] = c[1];
+        n.c1yz[1] = c[2];
+    }
+    for (int k = 0; k < 3; ++k) n.e[3 * slot + k] = half_up(e[k]);
+    n.ref[slot] = ref;
+}
+
 inline void set_child(BvhNode& n, int slot, const Box& b, uint32_t ref)
 {
     float c[3], e[3];
     for (int k = 0; k < 3; ++k) centre_extent(b.lo[k], b.hi[k], c[k], e[k]);
-    if (slot == 0) {
-        n.a[0] = c[0]; n.a[1] = e[0]; n.a[2] = c[1]; n.a[3] = e[1];
-        n.b[0] = c[2]; n.b[1] = e[2];
-    } else {
-        n.b[2] = c[0]; n.b[3] = e[0];
-        n.c[0] = c[1]; n.c[1] = e[1]; n.c[2] = c[2]; n.c[3] = e[2];
-    }
-    n.d[slot] = ref;
+    put_box(n, slot, c, e, ref);
 }
 
 // A child box every ray enters (centre 0, infinite extent).
 inline void set_child_always(BvhNode& n, int slot, uint32_t ref)
 {
     const float inf = std::numeric_limits<float>::infinity();
-    if (slot == 0) {
-        n.a[0] = 0.0f; n.a[1] = inf; n.a[2] = 0.0f; n.a[3] = inf;
-        n.b[0] = 0.0f; n.b[1] = inf;
-    } else {
-        n.b[2] = 0.0f; n.b[3] = inf;
-        n.c[0] = 0.0f; n.c[1] = inf; n.c[2] = 0.0f; n.c[3] = inf;
-    }
-    n.d[slot] = ref;
+    const float c[3] = {0.0f, 0.0f, 0.0f}, e[3] = {inf, inf, inf};
+    put_box(n, slot, c, e, ref);
 }
 
 // A child box no ray enters (the point (1e30, 1e30, 1e30)).
 inline void set_child_never(BvhNode& n, int slot, uint32_t ref)
 {
-    if (slot == 0) {
-        n.a[0] = kEmpty; n.a[1] = 0.0f; n.a[2] = kEmpty; n.a[3] = 0.0f;
-        n.b[0] = kEmpty; n.b[1] = 0.0f;
-    } else {
-        n.b[2] = kEmpty; n.b[3] = 0.0f;
-        n.c[0] = kEmpty; n.c[1] = 0.0f; n.c[2] = kEmpty; n.c[3] = 0.0f;
-    }
-    n.d[slot] = ref;
+    const float c[3] = {kEmpty, kEmpty, kEmpty}, e[3] = {0.0f, 0.0f, 0.0f};
+    put_box(n, slot, c, e, ref);
 }
 
 struct Builder {
@@ -265,12 +259,12 @@ struct Builder {
         }
         set_child(s.nodes[idx], 0, lb, lref);
         set_child(s.nodes[idx], 1, rb, rref);
-        return idx;
+        return inner_ref(idx);
     }
 
     static uint32_t fix(uint32_t ref, uint32_t node_off, uint32_t tri_off, uint32_t sph_off)
     {
-        if (!(ref & kRefLeaf)) return ref + node_off;
+        if (!(ref & kRefLeaf)) return ref + inner_ref(node_off);
         const uint32_t first = (ref & kRefFirstMask) + ((ref & kRefSphere) ? sph_off : tri_off);
         return (ref & ~kRefFirstMask) | first;
     }
@@ -282,8 +276,8 @@ struct Builder {
         const uint32_t tri_off = (uint32_t)s.tri_ids.size();
         const uint32_t sph_off = (uint32_t)s.sph_ids.size();
         for (BvhNode nd : r.nodes) {
-            nd.d[0] = fix(nd.d[0], node_off, tri_off, sph_off);
-            nd.d[1] = fix(nd.d[1], node_off, tri_off, sph_off);
+            nd.ref[0] = fix(nd.ref[0], node_off, tri_off, sph_off);
+            nd.ref[1] = fix(nd.ref[1], node_off, tri_off, sph_off);
             s.nodes.push_back(nd);
         }
         s.tri_ids.insert(s.tri_ids.end(), r.tri_ids.begin(), r.tri_ids.end());
@@ -329,7 +323,7 @@ void offset_inner_refs(std::vector<BvhNode>& nodes, uint32_t off)
 {
     for (BvhNode& n : nodes)
         for (int s = 0; s < 2; ++s)
-            if (!(n.d[s] & kRefLeaf)) n.d[s] += off;
+            if (!(n.ref[s] & kRefLeaf)) n.ref[s] += inner_ref(off);
 }
 
 BuildOutput build_bvh(const BuildInput& in)
@@ -398,6 +392,9 @@ BuildOutput build_bvh(const BuildInput& in)
             r2 = std::max(r2, d2);
         }
         out.sph_r = (float)(std::sqrt(r2) * (1.0 + 1e-6) + 1e-6);
+        out.sph_rmin = std::numeric_limits<float>::infinity();
+        for (size_t i = n_tri; i < prims.size(); ++i)
+            out.sph_rmin = std::min(out.sph_rmin, std::fabs(in.sph[(size_t)prims[i].id * 16 + 15]));
     }
 
     Sub s;
@@ -430,10 +427,7 @@ BuildOutput build_bvh(const BuildInput& in)
         s.depth = std::max(s.depth, 1u);
     }
     if (out.sph_node0 != 0xFFFFFFFFu) {
-        const float one = 1.0f;
-        uint32_t m;
-        std::memcpy(&m, &one, sizeof m);
-        for (size_t i = out.sph_node0; i < s.nodes.size(); ++i) s.nodes[i].d[2] = m;
+        for (size_t i = out.sph_node0; i < s.nodes.size(); ++i) s.nodes[i].m = 1.0f;
     }
     out.nodes = std::move(s.nodes);
     out.leaves = s.leaves;

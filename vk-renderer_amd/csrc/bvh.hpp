@@ -6,15 +6,15 @@
 // from the hits it reports (see trace_kernels.hip).
 //
 // Layout (all records 16-byte aligned for 128-bit loads):
-//   Node (64 B): the bounds of BOTH children, as centre and half-extent per
-//   axis (rounded so the float box contains the exact one), plus their refs,
-//   so one node fetch tests two boxes:
-//     a = (c0.cx, c0.ex, c0.cy, c0.ey)
-//     b = (c0.cz, c0.ez, c1.cx, c1.ex)
-//     c = (c1.cy, c1.ey, c1.cz, c1.ez)
-//     d = (ref0, ref1, m, 0)
-//   m is the float 1.0 in the nodes of the sphere subtree and 0 elsewhere;
-//   the traversal multiplies its per-ray widening by it.
+//   Node (48 B): the bounds of BOTH children, as centre and half-extent per
+//   axis, plus their refs, so one node fetch tests two boxes.  Centres are
+//   floats, half-extents 16-bit floats rounded up (the kernels' mixed
+//   multiply-add reads them as they are), so that [c - e, c + e] contains the
+//   float box; no half-extent is below 2^-14.  m is the float 1.0 in the nodes
+//   of the sphere subtree and 0 elsewhere; the traversal multiplies its
+//   per-ray widening by it.  Three 128-bit loads instead of the four that
+//   32-bit half-extents need: with several emitters the traversal is bound by
+//   the L1's address rate (97% of its cycles: each lane's load counts).
 //   With a centre/extent box the slab test is t = (c - o) / d -+ e / |d|, and
 //   a per-ray widening w of the box is one more term: (e + w) / |d|.
 //   Triangles and spheres live in separate subtrees: when both exist, node 0
@@ -24,14 +24,17 @@
 //   sphere subtree per ray (the reference's sphere test is imprecise far from
 //   the sphere, see traverse.hpp).
 //   ref: bit31 = leaf; for a leaf bit30 = sphere leaf, bits 27..29 = count-1,
-//   bits 0..26 = first record; for an inner node the node index.
+//   bits 0..26 = first record; for an inner node 3 * the node index (its
+//   offset in units of 16 bytes).
 //   Triangle record (48 B): (v0, key) (e1, mat_index) (e2, 0) where
 //   e1 = fl(v1 - v0), e2 = fl(v2 - v0) are exactly the edges the reference
 //   computes (Tracer.comp:342-343) and key is the triangle's scan index.
 //   Sphere record (16 B + 4 B key): (centre, r) and the sphere's scan index.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
+#include <cstring>
 #include <vector>
 
 namespace vkr {
@@ -55,10 +58,14 @@ inline uint32_t default_leaf(uint32_t n_emitters) { return n_emitters >= 2u ? 1u
 constexpr uint32_t kDefaultMaxDepth = 23;
 
 struct alignas(16) BvhNode {
-    float a[4], b[4], c[4];
-    uint32_t d[4];
+    float c0[3], c1x;         // child 0's centre, child 1's x
+    float c1yz[2];
+    uint32_t ref[2];
+    uint16_t e[6];            // half-extents: child 0 x y z, child 1 x y z
+    float m;
 };
-static_assert(sizeof(BvhNode) == 64, "node is 64 bytes");
+static_assert(sizeof(BvhNode) == 48, "node is 48 bytes");
+inline uint32_t inner_ref(std::size_t index) { return 3u * (uint32_t)index; }
 
 struct alignas(16) TriRecord {
     float v0[3]; uint32_t key;
@@ -66,6 +73,20 @@ struct alignas(16) TriRecord {
     float e2[3]; uint32_t pad;
 };
 static_assert(sizeof(TriRecord) == 48, "triangle record is 48 bytes");
+
+// The least 16-bit float >= x, for x >= 0 (above 65504: infinity), but at
+// least 2^-14, the smallest normal one.
+#if defined(__HIP__)
+__host__ __device__
+#endif
+inline uint16_t half_up(float x)
+{
+    if (!(x > 0x1p-14f)) return 0x0400u;
+    if (x > 65504.0f) return 0x7C00u;
+    uint32_t u;
+    memcpy(&u, &x, sizeof u);
+    return (uint16_t)(((u >> 13) - (112u << 10)) + ((u & 0x1FFFu) ? 1u : 0u));
+}
 
 struct BuildInput {
     const float* tri_v;       // n_tris * 12 floats: v0(3) pad v1(3) pad v2(3) pad (std430)
@@ -88,6 +109,7 @@ struct BuildOutput {
     uint32_t sph_node0 = 0xFFFFFFFFu;  // first node of the sphere subtree (none: all ones)
     float sph_c[3] = {0.0f, 0.0f, 0.0f};  // sphere centres lie within sph_r of sph_c
     float sph_r = 0.0f;
+    float sph_rmin = 0.0f;         // least radius
     bool empty = true;
 };
 
@@ -96,7 +118,7 @@ struct BuildOutput {
 // tri_ref, child 1 always entered with ref sph_ref.
 BvhNode join_root(const float lo[3], const float hi[3], uint32_t tri_ref, uint32_t sph_ref);
 
-// Adds off to every inner-node ref of nodes (leaf refs are unchanged).
+// Moves every inner-node ref of nodes by off nodes (leaf refs are unchanged).
 void offset_inner_refs(std::vector<BvhNode>& nodes, uint32_t off);
 
 // Builds a binned-SAH BVH.  Leaves hold one primitive kind only and at most

@@ -29,6 +29,7 @@ struct DevScene {
     uint32_t n_materials, flags, has_bvh, stack_needed;
     uint32_t emitters_bounded;      // every emitter: |emissive| < 2^20, 2^-20 <= r <= 2^20
     float sph_c[3], sph_r;          // every sphere centre lies within sph_r of sph_c
+    float sph_rmin;                 // the least radius
     // Scenes of a few primitives, traced by scanning (scan.hpp, use_scan).
     uint32_t scan;                  // 1: the scan records exist
     float scan_reach;               // sph_r + the largest radius
@@ -123,8 +124,7 @@ constexpr uint32_t kMaxPlainLanes = 1u << 21;
 //            traces (acc, u) (mask, v) (e, random-stream position) and, once
 //            per pixel, (bits of the primary hit's primitive, its t, -, -),
 //            at kWPark + 1024 i
-//   kWHead   the origin xyz of this step's rays; w holds the bits of the job
-//            (index in the batch, 0 for a single frame)
+//   kWHead   the origin xyz of this step's rays
 //   kWSlotD  per slot: the ray's (d xyz, t_max)
 //   kWSlotC  per slot: the next-event contribution (xyz, 0); slot 0 (a
 //            segment has none) holds kWPix, the sum of the pixel's finished

@@ -90,12 +90,13 @@ __device__ __forceinline__ void put_child_box(BvhNode* n, int slot, const float*
         }
     }
     if (slot == 0) {
-        n->a[0] = c[0]; n->a[1] = e[0]; n->a[2] = c[1]; n->a[3] = e[1];
-        n->b[0] = c[2]; n->b[1] = e[2];
+        for (int k = 0; k < 3; ++k) n->c0[k] = c[k];
     } else {
-        n->b[2] = c[0]; n->b[3] = e[0];
-        n->c[0] = c[1]; n->c[1] = e[1]; n->c[2] = c[2]; n->c[3] = e[2];
+        n->c1x = c[0];
+        n->c1yz[0] = c[1];
+        n->c1yz[1] = c[2];
     }
+    for (int k = 0; k < 3; ++k) n->e[3 * slot + k] = half_up(e[k]);
 }
 
 // Block-wide min (k < 3) / max (k >= 3) of six ordered values; thread 0
@@ -240,17 +241,16 @@ __global__ __launch_bounds__(kBuildBlock) void k_topology(int n, const uint64_t*
     // leaf (and not a Karras internal node).
     const uint32_t nl = (uint32_t)(g - lo + 1), nr = (uint32_t)(hi - g);
     const uint32_t r0 = nl <= max_leaf ? (kRefLeaf | ((nl - 1u) << kRefCountShift) | (uint32_t)lo)
-                                       : node_off + (uint32_t)g;
+                                       : 3u * (node_off + (uint32_t)g);
     const uint32_t r1 = nr <= max_leaf ? (kRefLeaf | ((nr - 1u) << kRefCountShift) | (uint32_t)(g + 1))
-                                       : node_off + (uint32_t)(g + 1);
+                                       : 3u * (node_off + (uint32_t)(g + 1));
     if (nl > 1u) par_in[g] = (uint32_t)i;
     if (nr > 1u) par_in[g + 1] = (uint32_t)i;
     alive[i] = (i == 0 || (uint32_t)(hi - lo + 1) > max_leaf) ? 1u : 0u;
     BvhNode* nd = nodes + node_off + i;
-    nd->d[0] = r0;
-    nd->d[1] = r1;
-    nd->d[2] = 0u;   // m = 0: triangle subtree, no per-ray widening
-    nd->d[3] = 0u;
+    nd->ref[0] = r0;
+    nd->ref[1] = r1;
+    nd->m = 0.0f;   // triangle subtree: no per-ray widening
 }
 
 constexpr uint32_t kDepthLimit = 255;   // deeper trees are reported as 255 (and rejected)
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_depth(uint32_t ni, uint32_t nod
             const BvhNode& nd = nodes[node_off + i];
             v[0] = d;
             v[1] = 1u;
-            v[2] = ((nd.d[0] & kRefLeaf) ? 1u : 0u) + ((nd.d[1] & kRefLeaf) ? 1u : 0u);
+            v[2] = ((nd.ref[0] & kRefLeaf) ? 1u : 0u) + ((nd.ref[1] & kRefLeaf) ? 1u : 0u);
         } else {
             depth[i] = kDead;
         }
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(kBuildBlock) void k_level(uint32_t ni, uint32_t lev
     float lo[3] = {__builtin_huge_valf(), __builtin_huge_valf(), __builtin_huge_valf()};
     float hi[3] = {-__builtin_huge_valf(), -__builtin_huge_valf(), -__builtin_huge_valf()};
     for (int slot = 0; slot < 2; ++slot) {
-        const uint32_t ref = nd->d[slot];
+        const uint32_t ref = nd->ref[slot];
         float4 l, h;
         if (ref & kRefLeaf) {
             const uint32_t first = ref & kRefFirstMask, cnt = ((ref >> kRefCountShift) & 7u) + 1u;
@@ -358,8 +358,8 @@ __global__ __launch_bounds__(kBuildBlock) void k_level(uint32_t ni, uint32_t lev
                 h = make_float4(fmaxf(h.x, h2.x), fmaxf(h.y, h2.y), fmaxf(h.z, h2.z), 0.0f);
             }
         } else {
-            l = nlo[ref - node_off];
-            h = nhi[ref - node_off];
+            l = nlo[ref / 3u - node_off];
+            h = nhi[ref / 3u - node_off];
         }
         const float cl[3] = {l.x, l.y, l.z}, ch[3] = {h.x, h.y, h.z};
         put_child_box(nd, slot, cl, ch);

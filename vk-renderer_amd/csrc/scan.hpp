@@ -212,6 +212,29 @@ __device__ __forceinline__ TravOut scan_ray(const DevScene& sc, f3 o, f3 d, floa
     return r;
 }
 
+// The wave's queued rays, as traverse_pool takes them: 64 at a time.
+__device__ __forceinline__ void scan_pool(const JobDesc& j, uint32_t total, const uint32_t* cpre,
+                                          const unsigned long long* colm, uint32_t* occ, uint2* res,
+                                          const char* __restrict__ wrec)
+{
+    for (uint32_t base = 0; base < total; base += 64u) {
+        const uint32_t i = base + __lane_id();
+        const bool act = i < total;
+        uint32_t slot = 0, lo = 0;
+        float4 h{}, r{};
+        if (act) {
+            pool_item(cpre, colm, i, slot, lo);
+            h = *reinterpret_cast<const float4*>(wrec + (kWHead + lo * 16u));
+            r = *reinterpret_cast<const float4*>(wrec + (kWSlotD + (slot * 64u + lo) * 16u));
+        }
+        const TravOut t = scan_ray(j.sc, f3{h.x, h.y, h.z}, f3{r.x, r.y, r.z}, r.w, j.eps, slot != 0u, act);
+        if (act) {
+            if (slot == 0u) res[lo] = make_uint2(t.prim, __float_as_uint(t.t));
+            else if (t.hit) atomicOr(occ + lo, 1u << slot);
+        }
+    }
+}
+
 // A shadow ray (sh) and a path segment (seg) from one origin, as traverse_pair.
 __device__ __forceinline__ TravOut scan_pair(const DevScene& sc, f3 o, bool sh, f3 sd, float st, bool seg, f3 d,
                                              float tmax, float eps, bool& occluded)

@@ -44,15 +44,17 @@ __device__ __forceinline__ const JobDesc& uniform_job(unsigned long long at)
     return *(const JobDesc*)reinterpret_cast<const __attribute__((address_space(4))) JobDesc*>(at);
 }
 
-// Runs body(job) with a job that is the same for all running lanes: once for a
-// launch of one job, else once for each job that the wave's lanes hold (one,
-// but for the few waves at a job's edge).
+// Runs body(job, mine) with a uniform job: once for a launch of one job, else
+// once for each job that the wave's lanes hold (one, but for the waves at a
+// job's edge); mine: the lane's own.  All lanes run it.  With a job of its own
+// in every lane instead, the scene's pointers would be per-lane values that
+// each node fetch loads, or holds eight registers for.
 template <bool BATCH, class Body>
 __device__ __forceinline__ void for_each_job(const PathLaunch& A, unsigned long long job_at, uint32_t job, bool active,
                                              Body&& body)
 {
     if constexpr (!BATCH) {
-        body(uniform_job(job_at));
+        body(uniform_job(job_at), true);
     } else {
         unsigned long long todo = __ballot(active);
         while (todo) {
@@ -62,7 +64,7 @@ __device__ __forceinline__ void for_each_job(const PathLaunch& A, unsigned long 
             const unsigned long long at = (unsigned long long)(A.jobs + j);
             const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
             const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
-            if (mine) body(uniform_job(((unsigned long long)hi << 32) | lo));
+            body(uniform_job(((unsigned long long)hi << 32) | lo), mine);
         }
     }
 }
@@ -300,14 +302,14 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
         if constexpr (!POOL) {
             // (3) At most a shadow ray and a segment per lane, from registers.
             bool occluded = false;
-            if constexpr (SCAN) {
-                for_each_job<BATCH>(A, job_at, job, has, [&](const JobDesc& jt) __attribute__((always_inline)) {
+            for_each_job<BATCH>(A, job_at, job, has, [&](const JobDesc& jt, bool mine) __attribute__((always_inline)) {
+                if (!mine) return;
+                if constexpr (SCAN)
                     tr = scan_pair(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, occluded);
-                });
-            } else {
-                const JobDesc& jt = BATCH ? A.jobs[job] : uniform_job(job_at);
-                tr = traverse_pair<BLOCK, COUNT>(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, stk, wc, occluded);
-            }
+                else
+                    tr = traverse_pair<BLOCK, COUNT>(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, stk, wc,
+                                                     occluded);
+            });
             if (sh && !occluded) e = add(e, c0);                     // :473, :502
         } else {
             // Path state that the wave's evaluation and tracing do not need
@@ -316,99 +318,73 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
             park[0] = make_float4(acc.x, acc.y, acc.z, uvx);
             park[64] = make_float4(mask.x, mask.y, mask.z, uvy);
             park[128] = make_float4(e.x, e.y, e.z, salt);
-            *reinterpret_cast<float4*>(wrec + (kWHead + lo16)) =
-                make_float4(ro.x, ro.y, ro.z, __uint_as_float(BATCH ? job : 0u));
+            *reinterpret_cast<float4*>(wrec + (kWHead + lo16)) = make_float4(ro.x, ro.y, ro.z, 0.0f);
             *reinterpret_cast<float4*>(wrec + (kWSlotD + lo16)) = make_float4(rd.x, rd.y, rd.z, tmax);
-            // The wave evaluates every published (lane, emitter) pair, slot
-            // by slot (neighbouring lanes take one emitter of neighbouring
-            // owners, whose records are neighbours).  A nonzero contribution
-            // goes to slot k of the owner (emitter ei0 + k - 1) and sets bit
-            // k of its mask.
-            const uint32_t tot = pool_columns(((1u << nitem) - 1u) << 1u, s_cpre + wslot, s_colm + wslot);
             s_msk[threadIdx.x] = has && seg ? 1u : 0u;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            for (uint32_t base = 0; base < tot; base += 64u) {
-                const uint32_t i = base + __lane_id();
-                if (i < tot) {
-                    uint32_t k, lo;
-                    pool_item(s_cpre + wslot, s_colm + wslot, i, k, lo);
-                    const uint32_t oo = lo * 16u;
-                    const float4 hd = *reinterpret_cast<const float4*>(wrec + (kWHead + oo));
-                    const float4 h0 = *reinterpret_cast<const float4*>(wrec + (kWHit + oo));
-                    const float4 h1 = *reinterpret_cast<const float4*>(wrec + (kWHit + 1024u + oo));
-                    const float4 h2 = *reinterpret_cast<const float4*>(wrec + (kWHit + 2048u + oo));
-                    const float4 h3 = *reinterpret_cast<const float4*>(wrec + (kWHit + 3072u + oo));
-                    const float sk = *reinterpret_cast<const float*>(wrec + (kWSalt + (k * 64u + lo) * 4u));
-                    const JobDesc& oj = BATCH ? A.jobs[__float_as_uint(hd.w)] : uniform_job(job_at);
-                    NeeHit h;
-                    h.P = f3{hd.x, hd.y, hd.z};
-                    h.N = f3{h0.x, h0.y, h0.z};
-                    h.V = f3{h2.x, h2.y, h2.z};
-                    h.alb = f3{h1.x, h1.y, h1.z};
-                    h.rough = h1.w;
-                    h.metal = h2.w;
-                    h.flags = __float_as_uint(h3.x);
-                    f3 L, c;
-                    float tl;
-                    if (nee_sample(oj, h, __float_as_uint(h3.z) + k - 1u, sk, h0.w, h3.y, L, tl, c)) {
-                        const uint32_t so = (k * 64u + lo) * 16u;
-                        *reinterpret_cast<float4*>(wrec + (kWSlotD + so)) = make_float4(L.x, L.y, L.z, tl);
-                        *reinterpret_cast<float4*>(wrec + (kWSlotC + so)) = make_float4(c.x, c.y, c.z, 0.0f);
-                        atomicOr(s_msk + wbase + lo, 1u << k);
-                    }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // (3) The wave traces all queued rays together from its pool, slot
-            // by slot: column k holds slot k of every lane that queued one,
-            // lanes in order.  Neighbouring lanes then take rays of one slot
-            // (the path segments, or one emitter) from neighbouring pixels,
-            // which visit much the same nodes.
-            const uint32_t msk = s_msk[threadIdx.x];
-            c_traced += (uint32_t)__popc(msk & ~1u);
-            const uint32_t nrays = pool_columns(msk, s_cpre + wslot, s_colm + wslot);
             s_occ[threadIdx.x] = 0u;
-            // The pool, the records and the result words are shared by the
-            // wave's lanes: order the writes above before the reads below.
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if constexpr (SCAN) {
-                for (uint32_t base = 0; base < nrays; base += 64u) {
+            auto fence = []() __attribute__((always_inline)) {
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            };
+            for_each_job<BATCH>(A, job_at, job, has, [&](const JobDesc& jt, bool mine) __attribute__((always_inline)) {
+                // The wave evaluates every published (lane, emitter) pair,
+                // slot by slot (neighbouring lanes take one emitter of
+                // neighbouring owners, whose records are neighbours).  A
+                // nonzero contribution goes to slot k of the owner (emitter
+                // ei0 + k - 1) and sets bit k of its mask.
+                const uint32_t tot = pool_columns(mine ? ((1u << nitem) - 1u) << 1u : 0u, s_cpre + wslot, s_colm + wslot);
+                fence();
+                for (uint32_t base = 0; base < tot; base += 64u) {
                     const uint32_t i = base + __lane_id();
-                    const bool act = i < nrays;
-                    uint32_t k = 0, lo = 0, rj = 0;
-                    f3 o{}, d{};
-                    float tm = 0.0f;
-                    if (act) {
+                    if (i < tot) {
+                        uint32_t k, lo;
                         pool_item(s_cpre + wslot, s_colm + wslot, i, k, lo);
-                        const float4 h = *reinterpret_cast<const float4*>(wrec + (kWHead + lo * 16u));
-                        const float4 r = *reinterpret_cast<const float4*>(wrec + (kWSlotD + (k * 64u + lo) * 16u));
-                        o = f3{h.x, h.y, h.z};
-                        rj = __float_as_uint(h.w);
-                        d = f3{r.x, r.y, r.z};
-                        tm = r.w;
-                    }
-                    TravOut t{kMiss, 0.0f, false};
-                    for_each_job<BATCH>(A, job_at, rj, act, [&](const JobDesc& jt) __attribute__((always_inline)) {
-                        t = scan_ray(jt.sc, o, d, tm, jt.eps, k != 0u, act);
-                    });
-                    if (act) {
-                        if (k == 0u) s_res[wbase + lo] = make_uint2(t.prim, __float_as_uint(t.t));
-                        else if (t.hit) atomicOr(s_occ + wbase + lo, 1u << k);
+                        const uint32_t oo = lo * 16u;
+                        const float4 hd = *reinterpret_cast<const float4*>(wrec + (kWHead + oo));
+                        const float4 h0 = *reinterpret_cast<const float4*>(wrec + (kWHit + oo));
+                        const float4 h1 = *reinterpret_cast<const float4*>(wrec + (kWHit + 1024u + oo));
+                        const float4 h2 = *reinterpret_cast<const float4*>(wrec + (kWHit + 2048u + oo));
+                        const float4 h3 = *reinterpret_cast<const float4*>(wrec + (kWHit + 3072u + oo));
+                        const float sk = *reinterpret_cast<const float*>(wrec + (kWSalt + (k * 64u + lo) * 4u));
+                        NeeHit h;
+                        h.P = f3{hd.x, hd.y, hd.z};
+                        h.N = f3{h0.x, h0.y, h0.z};
+                        h.V = f3{h2.x, h2.y, h2.z};
+                        h.alb = f3{h1.x, h1.y, h1.z};
+                        h.rough = h1.w;
+                        h.metal = h2.w;
+                        h.flags = __float_as_uint(h3.x);
+                        f3 L, c;
+                        float tl;
+                        if (nee_sample(jt, h, __float_as_uint(h3.z) + k - 1u, sk, h0.w, h3.y, L, tl, c)) {
+                            const uint32_t so = (k * 64u + lo) * 16u;
+                            *reinterpret_cast<float4*>(wrec + (kWSlotD + so)) = make_float4(L.x, L.y, L.z, tl);
+                            *reinterpret_cast<float4*>(wrec + (kWSlotC + so)) = make_float4(c.x, c.y, c.z, 0.0f);
+                            atomicOr(s_msk + wbase + lo, 1u << k);
+                        }
                     }
                 }
-            } else {
-                traverse_pool<BLOCK, COUNT, BATCH>(BATCH ? A.jobs : &uniform_job(job_at), nrays, s_cpre + wslot, s_colm + wslot,
-                                                   s_occ + wbase, s_res + wbase, wrec, stk, wc);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                fence();
+                // (3) The wave traces all queued rays together from its pool,
+                // slot by slot: column k holds slot k of every lane that
+                // queued one, lanes in order.  Neighbouring lanes then take
+                // rays of one slot (the path segments, or one emitter) from
+                // neighbouring pixels, which visit much the same nodes.
+                const uint32_t msk = mine ? s_msk[threadIdx.x] : 0u;
+                c_traced += (uint32_t)__popc(msk & ~1u);
+                const uint32_t nrays = pool_columns(msk, s_cpre + wslot, s_colm + wslot);
+                // The pool, the records and the result words are shared by
+                // the wave's lanes: order the writes above before the reads
+                // below.
+                fence();
+                if constexpr (SCAN)
+                    scan_pool(jt, nrays, s_cpre + wslot, s_colm + wslot, s_occ + wbase, s_res + wbase, wrec);
+                else
+                    traverse_pool<BLOCK, COUNT>(jt, nrays, s_cpre + wslot, s_colm + wslot, s_occ + wbase, s_res + wbase,
+                                                wrec, stk, wc);
+                fence();
+            });
             const float4 k0 = park[0], k1 = park[64], k2 = park[128];
             acc = f3{k0.x, k0.y, k0.z};
             mask = f3{k1.x, k1.y, k1.z};

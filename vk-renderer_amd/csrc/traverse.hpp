@@ -29,9 +29,8 @@ constexpr uint32_t kDone = 0xFFFFFFFFu;
 // 100k-triangle frames with leaves of at most 2 primitives (2/8 and 6/8 are
 // 12% and 4% slower with the pooled loop).
 constexpr uint32_t kLeafExit8 = 4;
-constexpr uint32_t kPhTrace = 0;
-constexpr uint32_t kPhNee = 1;
-constexpr int kCand = 4;
+
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 struct WorkCnt {
     uint32_t nodes, tris, spheres, planes, overflow;
@@ -59,6 +58,20 @@ __device__ __forceinline__ void cswap(float& ta, uint32_t& ka, float& tb, uint32
     ta = t0; tb = t1; ka = k0; kb = k1;
 }
 
+// What the node and leaf loops read.  Loaded once before them: a field of a
+// scene that is loaded where it is used (uniform_job) would put a scalar load
+// in front of every node fetch.
+struct TreePtrs {
+    const BvhNode* nodes;
+    const TriRecord* tris;
+    const float4* sph;
+    const uint32_t* sph_key;
+    __device__ __forceinline__ explicit TreePtrs(const DevScene& sc)
+        : nodes(sc.nodes), tris(sc.tris), sph(sc.sph), sph_key(sc.sph_key)
+    {
+    }
+};
+
 // One ray in flight: trace_ray of Assets/Tracer.comp:374-431 over the BVH.
 //   any == false: closest hit with the reference's acceptance rule.
 //   any == true : only "was anything accepted" (shadow rays, :473).
@@ -77,6 +90,14 @@ struct Ray {
     // here so that node steps do not recompute it (it changes only at leaves).
     __device__ __forceinline__ void set_cull(float cull) { cb = cull + fabsf(cull) * 1e-5f + 1e-5f; }
 
+    // 1 / d for the box test: the hardware's estimate and one Newton step.
+    __device__ __forceinline__ static float box_rcp(float d)
+    {
+        const float b = fabsf(d) > 1e-20f ? d : copysignf(1e-20f, d);
+        const float r = __builtin_amdgcn_rcpf(b);
+        return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+    }
+
     __device__ __forceinline__ void start(const DevScene& sc, f3 o_, f3 d_, float tmax_, float eps, bool any_)
     {
         const float inf = __builtin_huge_valf();
@@ -92,19 +113,24 @@ struct Ray {
         ovf = false;
         occluded = false;
         nan_ray = (d.x != d.x) || (d.y != d.y) || (d.z != d.z) || (o.x != o.x) || (o.y != o.y) || (o.z != o.z);
-        ix = 1.0f / (fabsf(d.x) > 1e-20f ? d.x : copysignf(1e-20f, d.x));
-        iy = 1.0f / (fabsf(d.y) > 1e-20f ? d.y : copysignf(1e-20f, d.y));
-        iz = 1.0f / (fabsf(d.z) > 1e-20f ? d.z : copysignf(1e-20f, d.z));
+        ix = box_rcp(d.x);
+        iy = box_rcp(d.y);
+        iz = box_rcp(d.z);
         ox = o.x * ix;
         oy = o.y * iy;
         oz = o.z * iz;
         // The sphere test (sphere_t, Assets/Tracer.comp:314-330) rounds its
-        // discriminant with an error up to ~60 ulp of |o - c|^2, so from far
-        // away it reports hits up to ~1e-3 |o - c| outside the sphere.  The
-        // sphere subtree's boxes are widened by 2e-3 (|o - C| + R), which
-        // bounds that distance for every centre c within R of C.
+        // discriminant, and the direction's length, with an error of up to
+        // 30u |o - c|^2 (u = 2^-24): it reports hits wherever the ray passes
+        // within r^2 + 30u |o - c|^2, squared, of the centre, and the reported
+        // point lies that near too.  So the sphere subtree's boxes are widened
+        // by w = sqrt(r^2 + 64u D^2) - r for the least radius r (w falls with
+        // r) and D >= |o - c| for every centre.
         const f3 oc = sub(o, f3{sc.sph_c[0], sc.sph_c[1], sc.sph_c[2]});
-        pad = fminf(2e-3f * (sqrtf(dot(oc, oc)) + sc.sph_r), 3e38f);
+        const float D = __builtin_amdgcn_sqrtf(dot(oc, oc)) + sc.sph_r;
+        const float q = 0x1p-18f * (D * D);
+        pad = q * __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(__builtin_fmaf(sc.sph_rmin, sc.sph_rmin, q)) + sc.sph_rmin);
+        pad = pad < 3e38f ? pad : 3e38f;   // (also from 0 / 0 and inf / inf)
         ref = (sc.has_bvh && !nan_ray) ? 0u : kDone;
         sp = 1;   // above the kDone entry the traversal loops keep at the bottom
     }
@@ -115,28 +141,33 @@ struct Ray {
     {
         // 32-bit byte offsets (node count < 2^26, checked at upload) let the
         // loads use a scalar base address.
-        const float4* np = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(nodes) + (ref << 6));
-        const float4 A = np[0], B = np[1], C = np[2];
-        const uint4 D = reinterpret_cast<const uint4*>(np)[3];
+        const float4* np = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(nodes) + (ref << 4));
+        const float4 A = np[0];                                  // child 0 centre, child 1 x
+        const float4 B = np[1];                                  // child 1 y z, refs
+        const float4 C = np[2];                                  // half-extents, m
+        const uint2 D{__float_as_uint(B.z), __float_as_uint(B.w)};
         if (COUNT) {
             wc.nodes++;
             count_wave(wc.wave_nodes);
         }
         // Slab test on centre/half-extent boxes: t = (c - o) i -+ (e + w) |i|,
         // with the widening w only in the sphere subtree (m = 1 there).
-        const float mp = __uint_as_float(D.z) * pad;
+        const half2_t e0 = __builtin_bit_cast(half2_t, C.x), e1 = __builtin_bit_cast(half2_t, C.y),
+                      e2 = __builtin_bit_cast(half2_t, C.z);
         const float ax = fabsf(ix), ay = fabsf(iy), az = fabsf(iz);
-        const float qx = mp * ax, qy = mp * ay, qz = mp * az;
-        const float a0 = __builtin_fmaf(A.x, ix, -ox), a1 = __builtin_fmaf(A.y, ax, qx);
-        const float a2 = __builtin_fmaf(A.z, iy, -oy), a3 = __builtin_fmaf(A.w, ay, qy);
-        const float a4 = __builtin_fmaf(B.x, iz, -oz), a5 = __builtin_fmaf(B.y, az, qz);
-        const float b0 = __builtin_fmaf(B.z, ix, -ox), b1 = __builtin_fmaf(B.w, ax, qx);
-        const float b2 = __builtin_fmaf(C.x, iy, -oy), b3 = __builtin_fmaf(C.y, ay, qy);
-        const float b4 = __builtin_fmaf(C.z, iz, -oz), b5 = __builtin_fmaf(C.w, az, qz);
-        const float n0 = fmaxf(fmaxf(a0 - a1, a2 - a3), fmaxf(a4 - a5, 0.0f));
-        const float f0 = fminf(fminf(a0 + a1, a2 + a3), fminf(a4 + a5, cb));
-        const float n1 = fmaxf(fmaxf(b0 - b1, b2 - b3), fmaxf(b4 - b5, 0.0f));
-        const float f1 = fminf(fminf(b0 + b1, b2 + b3), fminf(b4 + b5, cb));
+        const float ex0 = __builtin_fmaf(C.w, pad, (float)e0.x), ey0 = __builtin_fmaf(C.w, pad, (float)e0.y);
+        const float ez0 = __builtin_fmaf(C.w, pad, (float)e1.x), ex1 = __builtin_fmaf(C.w, pad, (float)e1.y);
+        const float ey1 = __builtin_fmaf(C.w, pad, (float)e2.x), ez1 = __builtin_fmaf(C.w, pad, (float)e2.y);
+        const float a0 = __builtin_fmaf(A.x, ix, -ox), a1 = __builtin_fmaf(A.y, iy, -oy), a2 = __builtin_fmaf(A.z, iz, -oz);
+        const float b0 = __builtin_fmaf(A.w, ix, -ox), b1 = __builtin_fmaf(B.x, iy, -oy), b2 = __builtin_fmaf(B.y, iz, -oz);
+        const float n0 = fmaxf(fmaxf(__builtin_fmaf(-ex0, ax, a0), __builtin_fmaf(-ey0, ay, a1)),
+                               fmaxf(__builtin_fmaf(-ez0, az, a2), 0.0f));
+        const float f0 = fminf(fminf(__builtin_fmaf(ex0, ax, a0), __builtin_fmaf(ey0, ay, a1)),
+                               fminf(__builtin_fmaf(ez0, az, a2), cb));
+        const float n1 = fmaxf(fmaxf(__builtin_fmaf(-ex1, ax, b0), __builtin_fmaf(-ey1, ay, b1)),
+                               fmaxf(__builtin_fmaf(-ez1, az, b2), 0.0f));
+        const float f1 = fminf(fminf(__builtin_fmaf(ex1, ax, b0), __builtin_fmaf(ey1, ay, b1)),
+                               fminf(__builtin_fmaf(ez1, az, b2), cb));
         const bool h0 = n0 <= f0, h1 = n1 <= f1;
         // The far child is always written to the free slot above the top
         // (sp < STACK at any inner node: the stack holds the kDone entry and
@@ -145,7 +176,7 @@ struct Ray {
         // children are hit.  With neither hit the top is popped; the bottom
         // kDone entry ends the traversal.
         const bool first0 = n0 <= n1;
-        const uint32_t nearr = (h0 && (!h1 || first0)) ? D.x : D.y;
+        const uint32_t nearr = (h1 && !(h0 && first0)) ? D.y : D.x;
         stk[sp * BLOCK] = first0 ? D.y : D.x;
         const uint32_t top = stk[(sp - 1) * BLOCK];
         const bool none = !h0 && !h1;
@@ -155,7 +186,7 @@ struct Ray {
 
     // Tests the primitives of leaf `ref`, then pops the stack.
     template <int BLOCK, bool COUNT>
-    __device__ __forceinline__ void leaf(const DevScene& sc, float eps, uint32_t* stk, WorkCnt& wc)
+    __device__ __forceinline__ void leaf(const TreePtrs& sc, float eps, uint32_t* stk, WorkCnt& wc)
     {
         const float inf = __builtin_huge_valf();
         const float win = 4.0f * eps;
@@ -169,6 +200,11 @@ struct Ray {
                 const float4 s4 = sc.sph[first + i];
                 if (COUNT) wc.spheres++;
                 t = sphere_t(o, d, f3{s4.x, s4.y, s4.z}, s4.w);
+                if (!(t > eps)) continue;
+                if (any) {   // (a shadow ray needs no key: the load is worth a branch)
+                    if (t < tmax_eps) occluded = true;
+                    continue;
+                }
                 key = 0x80000000u | sc.sph_key[first + i];
             } else {
                 const float4* tp = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(sc.tris) +
@@ -290,34 +326,6 @@ __device__ __forceinline__ bool leave_nodes(uint32_t nn, uint32_t nw)
     return nn == 0 || (nw > 0 && nw * 8u >= (nw + nn) * kLeafExit8);
 }
 
-// One ray per lane (lanes with active == false only take part in the
-// wave's loop).
-template <int BLOCK, bool COUNT>
-__device__ __forceinline__ TravOut traverse(const DevScene& sc, f3 o, f3 d, float tmax, float eps, bool any,
-                                            bool active, uint32_t* stk, WorkCnt& wc)
-{
-    Ray r;
-    r.start(sc, o, d, tmax, eps, any);
-    stk[0] = kDone;
-    if (!active) r.ref = kDone;
-    if (r.ref != kDone) {   // (only traversing lanes in the loop: 11 fewer VGPRs in k_path)
-        while (true) {
-            while (true) {
-                const uint32_t nn = (uint32_t)__popcll(__ballot((int)r.ref >= 0));
-                const uint32_t nl = (uint32_t)__popcll(__ballot((int)r.ref < -1));
-                if (leave_nodes(nn, nl)) break;
-                if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(sc.nodes, stk, wc);
-                if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(sc.nodes, stk, wc);
-            }
-            if (__ballot(r.ref != kDone) == 0) break;
-            if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(sc, eps, stk, wc);
-        }
-    }
-    // Lanes without a ray skip the plane list (their result is not read).
-    if (!active) return TravOut{kMiss, tmax, false};
-    return r.finish<COUNT>(sc, eps, wc);
-}
-
 // Whether a plane stops a shadow ray (the tests of Ray::finish; their order
 // does not matter to a yes or no).
 template <bool COUNT>
@@ -342,6 +350,7 @@ template <int BLOCK, bool COUNT>
 __device__ __forceinline__ TravOut traverse_pair(const DevScene& sc, f3 o, bool sh, f3 sd, float st, bool seg, f3 d,
                                                  float tmax, float eps, uint32_t* stk, WorkCnt& wc, bool& occluded)
 {
+    const TreePtrs tree(sc);
     occluded = sh && plane_stops<COUNT>(sc, o, sd, st, eps, wc);
     const bool first = sh && !occluded;
     bool next = first && seg;   // a segment waits behind the shadow ray
@@ -359,11 +368,11 @@ __device__ __forceinline__ TravOut traverse_pair(const DevScene& sc, f3 o, bool 
             const uint32_t nn = (uint32_t)__popcll(__ballot((int)r.ref >= 0));
             const uint32_t nw = (uint32_t)__popcll(__ballot((int)r.ref < -1 || (next && r.ref == kDone)));
             if (leave_nodes(nn, nw)) break;
-            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(sc.nodes, stk, wc);
-            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(sc.nodes, stk, wc);
+            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
+            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
         }
         if (__ballot(r.ref != kDone || next) == 0) break;
-        if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(sc, eps, stk, wc);
+        if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(tree, eps, stk, wc);
     }
     if (r.any) occluded = r.occluded;   // a shadow ray with no segment behind it
     if (!seg) return TravOut{kMiss, tmax, false};
@@ -433,14 +442,13 @@ __device__ __forceinline__ void pool_item(const uint32_t* cpre, const unsigned l
 // rays, which set bit `slot` of occ[owner] when occluded.  `wrec` is the wave's block of ray records
 // (kWHead, kWSlotD: the lanes of a wave reading one slot of neighbouring
 // owners read neighbouring addresses).
-template <int BLOCK, bool COUNT, bool BATCH>
-__device__ __forceinline__ void traverse_pool(const JobDesc* jobs, uint32_t total, const uint32_t* cpre,
+template <int BLOCK, bool COUNT>
+__device__ __forceinline__ void traverse_pool(const JobDesc& j, uint32_t total, const uint32_t* cpre,
                                               const unsigned long long* colm, uint32_t* occ, uint2* res,
                                               const char* __restrict__ wrec, uint32_t* stk, WorkCnt& wc)
 {
-    // The job (scene, epsilon) of the ray in flight: a batched wave can hold
-    // pixels of several jobs, and a lane may trace another lane's ray.
-    const JobDesc* rj = jobs;
+    const TreePtrs tree(j.sc);
+    const float eps = j.eps;
     Ray r;
     r.ref = kDone;
     stk[0] = kDone;
@@ -451,7 +459,7 @@ __device__ __forceinline__ void traverse_pool(const JobDesc* jobs, uint32_t tota
         // or the pool is empty.
         while (true) {
             if (cur != kNone && r.ref == kDone) {
-                const TravOut t = r.finish<COUNT>(rj->sc, rj->eps, wc);
+                const TravOut t = r.finish<COUNT>(j.sc, eps, wc);
                 const uint32_t owner = cur >> 5;
                 if (r.any) {
                     if (t.hit) atomicOr(occ + owner, 1u << (cur & 31u));
@@ -469,8 +477,7 @@ __device__ __forceinline__ void traverse_pool(const JobDesc* jobs, uint32_t tota
                     cur = (lo << 5) | slot;
                     const float4 h = *reinterpret_cast<const float4*>(wrec + (kWHead + lo * 16u));
                     const float4 s = *reinterpret_cast<const float4*>(wrec + (kWSlotD + (slot * 64u + lo) * 16u));
-                    if constexpr (BATCH) rj = jobs + __float_as_uint(h.w);   // the owner's job
-                    r.start(rj->sc, f3{h.x, h.y, h.z}, f3{s.x, s.y, s.z}, s.w, rj->eps, slot != 0u);
+                    r.start(j.sc, f3{h.x, h.y, h.z}, f3{s.x, s.y, s.z}, s.w, eps, slot != 0u);
                 }
                 next += (uint32_t)__popcll(want);
             }
@@ -482,10 +489,10 @@ __device__ __forceinline__ void traverse_pool(const JobDesc* jobs, uint32_t tota
             const uint32_t nn = (uint32_t)__popcll(__ballot((int)r.ref >= 0));
             const uint32_t nw = (uint32_t)__popcll(__ballot((int)r.ref < -1 || (more && r.ref == kDone)));
             if (leave_nodes(nn, nw)) break;
-            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(rj->sc.nodes, stk, wc);
-            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(rj->sc.nodes, stk, wc);
+            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
+            if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
         }
-        if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(rj->sc, rj->eps, stk, wc);
+        if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(tree, eps, stk, wc);
     }
 }
 

@@ -89,7 +89,7 @@ bool device_build(vkr_ctx* ctx, Scene* sc, uint32_t n, BuildInput bi, uint32_t d
 struct ScanPlan {
     bool ok = false;
     float r_max = 0.0f;
-    std::vector<float4> sph;
+    std::vector<float4> sph, planes;
     std::vector<TriRecord> tris;
 };
 
@@ -116,6 +116,15 @@ ScanPlan scan_plan(const vkr_scene_desc& d)
         r.key = i;
         p.tris.push_back(r);
     }
+    // Whole runs and one to read ahead: a sphere with r * r = -inf has no root,
+    // a plane with N = 0 no distance.
+    for (uint32_t i = 0; i < d.n_planes; ++i)
+        p.planes.push_back(make_float4(d.planes[i].N[0], d.planes[i].N[1], d.planes[i].N[2], d.planes[i].len));
+    const auto pad = [](std::vector<float4>& v, float4 none) {
+        v.resize((v.size() + kScanRun - 1u) / kScanRun * kScanRun + kScanRun, none);
+    };
+    pad(p.sph, make_float4(0.0f, 0.0f, 0.0f, -INFINITY));
+    pad(p.planes, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     p.ok = true;
     return p;
 }
@@ -276,6 +285,7 @@ vkr_error vkr_scene_upload(vkr_ctx* ctx, const vkr_scene_desc* desc, uint32_t* o
     const ScanPlan scan = scan_plan(*desc);
     if (scan.ok) {
         VKR_HIP(sc->scan_sph.upload(scan.sph.data(), scan.sph.size() * sizeof(float4)));
+        VKR_HIP(sc->scan_planes.upload(scan.planes.data(), scan.planes.size() * sizeof(float4)));
         VKR_HIP(sc->scan_tris.upload(scan.tris.data(), scan.tris.size() * sizeof(TriRecord)));
     }
 
@@ -305,6 +315,7 @@ vkr_error vkr_scene_upload(vkr_ctx* ctx, const vkr_scene_desc* desc, uint32_t* o
     d.scan = scan.ok ? 1u : 0u;
     d.scan_reach = bo.sph_r + scan.r_max;
     d.scan_sph = sc->scan_sph.as<float4>();
+    d.scan_planes = sc->scan_planes.as<float4>();
     d.scan_tris = sc->scan_tris.as<TriRecord>();
 
     sc->serial = ctx->next_serial++;

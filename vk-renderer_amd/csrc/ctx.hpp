@@ -73,7 +73,7 @@ const vkr_material kMirror = {{1.0f, 0.5f, 0.5f}, 0.0f, {0.0f, 0.0f, 0.0f}, 0.0f
 
 struct Scene {
     DevBuf nodes, tris, sph, sph_key, tris_orig, spheres, planes, tri_mat, materials, emitters;
-    DevBuf scan_sph, scan_tris;      // scenes that are scanned (scan.hpp)
+    DevBuf scan_sph, scan_tris, scan_planes;      // scenes that are scanned (scan.hpp)
     DevBuf theta;                    // device copy of the sphere parameters (adjoint)
     std::vector<vkr_sphere> host_spheres;
     std::vector<float> host_theta;   // 7 * n_spheres + 1

@@ -33,7 +33,8 @@ struct DevScene {
     // Scenes of a few primitives, traced by scanning (scan.hpp, use_scan).
     uint32_t scan;                  // 1: the scan records exist
     float scan_reach;               // sph_r + the largest radius
-    const float4* scan_sph;         // scan order: centre, r * r
+    const float4* scan_sph;         // scan order: centre, r * r; padded (kScanRun)
+    const float4* scan_planes;      // scan order: N, len; padded
     const TriRecord* scan_tris;     // scan order
 };
 
@@ -46,6 +47,9 @@ struct DevScene {
 //   1934 / 1754, 101: 3188 / 3014, 161: 5490 / 6450, but 512x512: 101: 1651 /
 //   1859;
 //   7 spheres and 16 triangles 350 / 306 us, 30 triangles 374 / 344.
+// Spheres and planes are read kScanRun at a time and padded to whole runs, plus
+// one that is read ahead, with primitives no ray hits.
+constexpr uint32_t kScanRun = 4u;
 constexpr uint32_t kScanUnits = 56u;       // single rays
 constexpr uint32_t kScanUnitsPool = 80u;   // ray pool
 inline uint32_t scan_units(uint32_t spheres, uint32_t tris)

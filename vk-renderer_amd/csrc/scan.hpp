@@ -34,6 +34,28 @@ typedef const __attribute__((address_space(4))) v4f* cv4f;
 
 __device__ __forceinline__ cv4f const_rows(const void* p) { return (cv4f) reinterpret_cast<unsigned long long>(p); }
 
+// Calls body(row, i) for rows 0 .. n - 1 of a padded array (the padding rows of
+// the last run included).  A run is loaded while the one before it is worked
+// on: a wave that has its SIMD to itself would otherwise wait out a scalar
+// load, as long as three sphere tests, for every row.
+template <class Body>
+__device__ __forceinline__ void for_rows(const void* rows, uint32_t n, Body&& body)
+{
+    const cv4f p = const_rows(rows);
+    v4f a = p[0], b = p[1], c = p[2], d = p[3];
+    for (uint32_t i = 0; i < n; i += kScanRun) {
+        const v4f a1 = p[i + 4u], b1 = p[i + 5u], c1 = p[i + 6u], d1 = p[i + 7u];
+        body(a, i);
+        body(b, i + 1u);
+        body(c, i + 2u);
+        body(d, i + 3u);
+        a = a1;
+        b = b1;
+        c = c1;
+        d = d1;
+    }
+}
+
 // The least two of a ray's hit distances beyond `lo`, and the least one's key.
 struct Nearest {
     float best, second;
@@ -98,12 +120,11 @@ __device__ __forceinline__ void scan_exact(const DevScene& sc, f3 o, f3 d, float
 __device__ __forceinline__ void scan_planes(const DevScene& sc, f3 o, f3 d, float eps, Nearest& n)
 {
     const float lo = eps * (1.0f - 0x1p-18f);
-    for (uint32_t i = 0; i < sc.n_planes; ++i) {
-        const v4f q = const_rows(sc.planes)[4u * i + 3u];   // (N, len)
+    for_rows(sc.scan_planes, sc.n_planes, [&](v4f q, uint32_t i) __attribute__((always_inline)) {
         const f3 N{q.x, q.y, q.z};
         const float num = q.w + dot(o, N);
         n.add(-num * __builtin_amdgcn_rcpf(dot(d, N)), lo, i);
-    }
+    });
 }
 
 // Whether a plane stops a shadow ray of length tmax (t in (eps, tmax - eps)).
@@ -200,11 +221,10 @@ __device__ __forceinline__ TravOut scan_ray(const DevScene& sc, f3 o, f3 d, floa
         const v4f a = p[0], b = p[1], c = p[2];
         n.add(tri_t(o, d, f3{a.x, a.y, a.z}, f3{b.x, b.y, b.z}, f3{c.x, c.y, c.z}, eps), eps, i);
     }
-    for (uint32_t i = 0; i < sc.n_spheres; ++i) {
-        const v4f s = const_rows(sc.scan_sph)[i];
+    for_rows(sc.scan_sph, sc.n_spheres, [&](v4f s, uint32_t i) __attribute__((always_inline)) {
         const f3 oc = sub(o, f3{s.x, s.y, s.z});
         n.add(SphereTerms(oc, dot(oc, oc) - s.w, d).near(), lo, (1u << 30) | i);
-    }
+    });
     TravOut r{kMiss, tmax, false};
     if (!active) return r;
     if (any) r.hit = scan_end_any(sc, o, d, tmax, eps, err, n) || scan_plane_stops(sc, o, d, tmax, eps);
@@ -250,13 +270,12 @@ __device__ __forceinline__ TravOut scan_pair(const DevScene& sc, f3 o, bool sh, 
         n.add(tri_t(o, d, v0, e1, e2, eps), eps, i);
         m.add(tri_t(o, sd, v0, e1, e2, eps), eps, i);
     }
-    for (uint32_t i = 0; i < sc.n_spheres; ++i) {
-        const v4f s = const_rows(sc.scan_sph)[i];
+    for_rows(sc.scan_sph, sc.n_spheres, [&](v4f s, uint32_t i) __attribute__((always_inline)) {
         const f3 oc = sub(o, f3{s.x, s.y, s.z});
         const float cc = dot(oc, oc) - s.w;
         n.add(SphereTerms(oc, cc, d).near(), lo, (1u << 30) | i);
         m.add(SphereTerms(oc, cc, sd).near(), lo, i);
-    }
+    });
     occluded = false;
     if (sh) occluded = scan_end_any(sc, o, sd, st, eps, err, m) || scan_plane_stops(sc, o, sd, st, eps);
     if (!seg) return TravOut{kMiss, tmax, false};

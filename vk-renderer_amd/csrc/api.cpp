@@ -89,22 +89,33 @@ bool device_build(vkr_ctx* ctx, Scene* sc, uint32_t n, BuildInput bi, uint32_t d
 struct ScanPlan {
     bool ok = false;
     float r_max = 0.0f;
-    std::vector<float4> sph, planes;
-    std::vector<TriRecord> tris;
+    std::vector<float4> rows;         // spheres, planes, triangles
+    size_t planes = 0, tris = 0;      // where they begin
 };
 
 ScanPlan scan_plan(const vkr_scene_desc& d)
 {
     ScanPlan p;
     if (scan_units(d.n_spheres, d.n_tris) > kScanUnitsPool) return p;
+    // Whole runs and one to read ahead.
+    const auto pad = [&p](size_t begin, float4 none) {
+        const size_t n = p.rows.size() - begin;
+        p.rows.resize(begin + (n + kScanRun - 1u) / kScanRun * kScanRun + kScanRun, none);
+    };
     for (uint32_t i = 0; i < d.n_spheres; ++i) {
         const vkr_sphere& s = d.spheres[i];
         for (int k = 0; k < 3; ++k)
             if (!(std::fabs(s.P[k]) < 0x1p40f)) return p;
         if (!(std::fabs(s.r) < 0x1p40f)) return p;
         p.r_max = std::max(p.r_max, std::fabs(s.r));
-        p.sph.push_back(make_float4(s.P[0], s.P[1], s.P[2], s.r * s.r));
+        p.rows.push_back(make_float4(s.P[0], s.P[1], s.P[2], s.r * s.r));
     }
+    pad(0, make_float4(0.0f, 0.0f, 0.0f, -INFINITY));   // r * r = -inf: no root
+    p.planes = p.rows.size();
+    for (uint32_t i = 0; i < d.n_planes; ++i)
+        p.rows.push_back(make_float4(d.planes[i].N[0], d.planes[i].N[1], d.planes[i].N[2], d.planes[i].len));
+    pad(p.planes, make_float4(0.0f, 0.0f, 0.0f, 0.0f));   // N = 0: no distance
+    p.tris = p.rows.size();
     for (uint32_t i = 0; i < d.n_tris; ++i) {
         const vkr_triangle& t = d.tris[i];
         TriRecord r{};
@@ -114,17 +125,10 @@ ScanPlan scan_plan(const vkr_scene_desc& d)
             r.e2[k] = t.v2[k] - t.v0[k];
         }
         r.key = i;
-        p.tris.push_back(r);
+        float4 rows[3];
+        std::memcpy(rows, &r, sizeof rows);
+        p.rows.insert(p.rows.end(), rows, rows + 3);
     }
-    // Whole runs and one to read ahead: a sphere with r * r = -inf has no root,
-    // a plane with N = 0 no distance.
-    for (uint32_t i = 0; i < d.n_planes; ++i)
-        p.planes.push_back(make_float4(d.planes[i].N[0], d.planes[i].N[1], d.planes[i].N[2], d.planes[i].len));
-    const auto pad = [](std::vector<float4>& v, float4 none) {
-        v.resize((v.size() + kScanRun - 1u) / kScanRun * kScanRun + kScanRun, none);
-    };
-    pad(p.sph, make_float4(0.0f, 0.0f, 0.0f, -INFINITY));
-    pad(p.planes, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     p.ok = true;
     return p;
 }
@@ -283,11 +287,7 @@ vkr_error vkr_scene_upload(vkr_ctx* ctx, const vkr_scene_desc* desc, uint32_t* o
     if (!em.empty()) VKR_HIP(hipMemcpy(sc->emitters.p, em.data(), em.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
 
     const ScanPlan scan = scan_plan(*desc);
-    if (scan.ok) {
-        VKR_HIP(sc->scan_sph.upload(scan.sph.data(), scan.sph.size() * sizeof(float4)));
-        VKR_HIP(sc->scan_planes.upload(scan.planes.data(), scan.planes.size() * sizeof(float4)));
-        VKR_HIP(sc->scan_tris.upload(scan.tris.data(), scan.tris.size() * sizeof(TriRecord)));
-    }
+    if (scan.ok) VKR_HIP(sc->scan.upload(scan.rows.data(), scan.rows.size() * sizeof(float4)));
 
     DevScene& d = sc->dev;
     d.nodes = sc->nodes.as<BvhNode>();
@@ -314,9 +314,9 @@ vkr_error vkr_scene_upload(vkr_ctx* ctx, const vkr_scene_desc* desc, uint32_t* o
     d.sph_rmin = bo.sph_rmin;
     d.scan = scan.ok ? 1u : 0u;
     d.scan_reach = bo.sph_r + scan.r_max;
-    d.scan_sph = sc->scan_sph.as<float4>();
-    d.scan_planes = sc->scan_planes.as<float4>();
-    d.scan_tris = sc->scan_tris.as<TriRecord>();
+    d.scan_sph = sc->scan.as<float4>();
+    d.scan_planes = d.scan_sph + scan.planes;
+    d.scan_tris = reinterpret_cast<const TriRecord*>(d.scan_sph + scan.tris);
 
     sc->serial = ctx->next_serial++;
     vkr_scene_info& in = sc->info;
@@ -509,7 +509,7 @@ static vkr_error plan_frame(vkr_ctx* ctx, uint32_t scene, const Scene& s, const 
     uint32_t& grid = f.grid;
     grid = (std::min(a.total, f.step) + block - 1u) / block;
     a.width = 64u;
-    if (persistent) persistent_shape(v, a.total, s.dev.n_emitters, ~0u, ctx->device, grid, a.width);
+    if (persistent) persistent_shape(v, a.total, s.dev, s.dev.n_emitters, ~0u, ctx->device, grid, a.width);
     if (v.pool) {
         const vkr_error le = ensure_lanes(ctx, (size_t)grid * block);
         if (le != VKR_SUCCESS) return le;
@@ -650,7 +650,7 @@ vkr_error vkr_trace_frame_static(vkr_ctx* ctx, uint32_t scene, const vkr_frame_d
             return fail(VKR_INVALID_ARGUMENT,
                         "VKR_SCHED_PLAIN with the ray pool needs one ray record per pixel, more than the static "
                         "scratch holds (VKR_STATIC_SCRATCH_LANE_BYTES); use the persistent schedule");
-        if (persistent) persistent_shape(v, a.total, s->dev.n_emitters, cap, ctx->device, grid, a.width);
+        if (persistent) persistent_shape(v, a.total, s->dev, s->dev.n_emitters, cap, ctx->device, grid, a.width);
         if (v.pool) {
             a.lanes = lanes;
         }

@@ -205,7 +205,7 @@ vkr_error vkr_trace_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n_jo
                                 cnt);
     const PathVariant v = batch_variant(plan, sh.block, count);
     uint32_t grid = 0, width = 64u;
-    persistent_shape(v, plan.total, plan.emitters, ~0u, ctx->device, grid, width);
+    persistent_shape(v, plan.total, plan.jobs[0].sc, plan.emitters, ~0u, ctx->device, grid, width);
     const vkr_error ce = check_cursor(plan, grid, sh.block);
     if (ce != VKR_SUCCESS) return ce;
     if (v.pool) {
@@ -237,7 +237,7 @@ vkr_error vkr_batch_graph_create(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32
     const BatchShape sh = batch_shape(ctx, jobs, n_jobs, plan, block, chunk);
     const PathVariant v = batch_variant(plan, sh.block, count);
     uint32_t grid = 0, width = 64u;
-    persistent_shape(v, plan.total, plan.emitters, ~0u, ctx->device, grid, width);
+    persistent_shape(v, plan.total, plan.jobs[0].sc, plan.emitters, ~0u, ctx->device, grid, width);
     const vkr_error ce = check_cursor(plan, grid, sh.block);
     if (ce != VKR_SUCCESS) return ce;
 

@@ -73,7 +73,7 @@ const vkr_material kMirror = {{1.0f, 0.5f, 0.5f}, 0.0f, {0.0f, 0.0f, 0.0f}, 0.0f
 
 struct Scene {
     DevBuf nodes, tris, sph, sph_key, tris_orig, spheres, planes, tri_mat, materials, emitters;
-    DevBuf scan_sph, scan_tris, scan_planes;      // scenes that are scanned (scan.hpp)
+    DevBuf scan;                     // scenes that are scanned (scan.hpp): spheres, planes, triangles
     DevBuf theta;                    // device copy of the sphere parameters (adjoint)
     std::vector<vkr_sphere> host_spheres;
     std::vector<float> host_theta;   // 7 * n_spheres + 1
@@ -304,15 +304,26 @@ inline bool use_ray_pool(uint32_t flags, uint32_t n_emitters)
 // 345 (8); 4 emitters 256^2 1021 -> 597 (16; 8: 648).  Single rays: 64^2
 // reference scene 102 -> 91 us (4), 64^2 16 spp adjoint scene 566 -> 517 (4),
 // but 256^2 563 -> 600 (32).
-inline void persistent_shape(const PathVariant& v, uint64_t total, uint32_t n_emitters, uint32_t max_grid, int device,
-                             uint32_t& grid, uint32_t& width)
+//
+// Single-ray waves of at most kQuadWidth pixels scan with four lanes a pixel
+// (scan.hpp).  So images that all fit such waves at once take 16 pixels a wave
+// if they fill no more than half of the lanes, or have kQuadUnits to test and
+// more: one pixel a lane against four (4 spp, depth 4), 9 units 160^2
+// 179 -> 170 us but 256^2 183 -> 227; 13 units 160^2 131 -> 120, 256x200
+// 127 -> 136; 33 units 160^2 182 -> 151, 256x200 177 -> 157, 256^2 166 -> 164;
+// 7 spheres and 16 triangles 160^2 215 -> 162, 256^2 228 -> 199.
+inline void persistent_shape(const PathVariant& v, uint64_t total, const DevScene& sc, uint32_t n_emitters,
+                             uint32_t max_grid, int device, uint32_t& grid, uint32_t& width)
 {
     const uint32_t waves = v.block / 64u;   // of a workgroup
     const uint32_t resident = std::min(persistent_grid(v, device), max_grid);
     const uint32_t simds = 4u * compute_units(device);
+    const uint64_t room = (uint64_t)kQuadWidth * resident * waves;
+    const bool quads = v.scan && !v.pool && !v.batch &&
+                       total <= (scan_units(sc.n_spheres, sc.n_tris) >= kQuadUnits ? room : room / 2u);
     const uint64_t rounds = v.pool ? std::min<uint64_t>(8u * simds, 2ull * resident * waves) : simds;
     const uint32_t least = v.pool ? (64u + std::max(n_emitters, 1u) - 1u) / std::max(n_emitters, 1u) : 1u;
-    width = 64u;
+    width = quads ? kQuadWidth : 64u;
     while (width / 2u >= least && total < rounds * width) width /= 2u;
     const uint64_t need = (total + (uint64_t)width * waves - 1u) / ((uint64_t)width * waves);
     grid = (uint32_t)std::max<uint64_t>(1u, std::min<uint64_t>(resident, need));

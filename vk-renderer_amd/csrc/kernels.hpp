@@ -52,6 +52,10 @@ struct DevScene {
 constexpr uint32_t kScanRun = 4u;
 constexpr uint32_t kScanUnits = 56u;       // single rays
 constexpr uint32_t kScanUnitsPool = 80u;   // ray pool
+// Single-ray waves of at most kQuadWidth pixels scan with four lanes a pixel;
+// kQuadUnits is part of the rule that gives a wave so few (ctx.hpp).
+constexpr uint32_t kQuadWidth = 16u;
+constexpr uint32_t kQuadUnits = 24u;
 inline uint32_t scan_units(uint32_t spheres, uint32_t tris)
 {
     return (uint32_t)std::min<uint64_t>((uint64_t)spheres + 2ull * tris, 0xFFFFFFFFull);

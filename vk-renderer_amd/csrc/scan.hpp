@@ -18,7 +18,8 @@
 //   * otherwise the lane runs the reference's own loop.
 // What bounds it: VALU issue.  Against the tree on the same kernels: 64^2
 // reference scene 127 -> 98 us, 1024^2 with present filter 1291 -> 1146 us,
-// 256^2, 16 spp, 33 spheres forward + backward 1536 -> 1154 us.
+// 256^2, 16 spp, 33 spheres forward + backward 1536 -> 1154 us.  The smallest
+// images are bound by a pixel's serial chain instead, see scan_pair_quad.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -37,7 +38,8 @@ __device__ __forceinline__ cv4f const_rows(const void* p) { return (cv4f) reinte
 // Calls body(row, i) for rows 0 .. n - 1 of a padded array (the padding rows of
 // the last run included).  A run is loaded while the one before it is worked
 // on: a wave that has its SIMD to itself would otherwise wait out a scalar
-// load, as long as three sphere tests, for every row.
+// load, as long as three sphere tests, for every row (65 spheres 512^2
+// 394 -> 369 us).
 template <class Body>
 __device__ __forceinline__ void for_rows(const void* rows, uint32_t n, Body&& body)
 {
@@ -127,12 +129,10 @@ __device__ __forceinline__ void scan_planes(const DevScene& sc, f3 o, f3 d, floa
     });
 }
 
-// Whether a plane stops a shadow ray of length tmax (t in (eps, tmax - eps)).
-__device__ __forceinline__ bool scan_plane_stops(const DevScene& sc, f3 o, f3 d, float tmax, float eps)
+// Whether a plane stops a shadow ray of length tmax (t in (eps, tmax - eps)), n
+// its planes from scan_planes.
+__device__ __forceinline__ bool scan_plane_stops(const DevScene& sc, f3 o, f3 d, float tmax, float eps, const Nearest& n)
 {
-    Nearest n;
-    n.clear();
-    scan_planes(sc, o, d, eps, n);
     const float lim = tmax - eps, slack = fabsf(lim) * 0x1p-18f;
     if (!(n.best < lim + slack)) return false;
     if (n.best > eps * (1.0f + 0x1p-18f) && n.best < lim - slack) return true;
@@ -140,12 +140,10 @@ __device__ __forceinline__ bool scan_plane_stops(const DevScene& sc, f3 o, f3 d,
     return plane_stops<false>(sc, o, d, tmax, eps, wc);
 }
 
-// The planes after triangles and spheres gave (best, prim).
-__device__ __forceinline__ void scan_plane_hits(const DevScene& sc, f3 o, f3 d, float eps, float& best, uint32_t& prim)
+// The planes (n, from scan_planes) after triangles and spheres gave (best, prim).
+__device__ __forceinline__ void scan_plane_hits(const DevScene& sc, f3 o, f3 d, float eps, const Nearest& n, float& best,
+                                                uint32_t& prim)
 {
-    Nearest n;
-    n.clear();
-    scan_planes(sc, o, d, eps, n);
     const float lim = best - eps, slack = (fabsf(best) + eps) * 0x1p-18f;
     if (!(n.best < lim + slack)) return;
     if (n.best > eps * (1.0f + 0x1p-18f) && n.best < lim - slack && n.second > n.best + eps + eps + slack) {
@@ -187,12 +185,12 @@ __device__ __forceinline__ bool scan_end_any(const DevScene& sc, f3 o, f3 d, flo
     scan_exact(sc, o, d, tmax, eps, true, t, key);
     return key != kMiss;
 }
-__device__ __forceinline__ TravOut scan_end_closest(const DevScene& sc, f3 o, f3 d, float tmax, float eps, float err,
-                                                    const Nearest& n)
+__device__ __forceinline__ void scan_end_closest(const DevScene& sc, f3 o, f3 d, float tmax, float eps, float err,
+                                                 const Nearest& n, float& best, uint32_t& prim)
 {
     const float lim = tmax + eps;
-    float best = tmax;
-    uint32_t prim = kMiss;
+    best = tmax;
+    prim = kMiss;
     if (!(n.best >= lim + err)) {
         if (n.best > eps + err && n.best < lim - err && !(n.second < n.best + (eps + 2.0f * err))) {
             prim = n.key;
@@ -206,8 +204,6 @@ __device__ __forceinline__ TravOut scan_end_closest(const DevScene& sc, f3 o, f3
             scan_exact(sc, o, d, tmax, eps, false, best, prim);
         }
     }
-    scan_plane_hits(sc, o, d, eps, best, prim);
-    return TravOut{prim, best, prim != kMiss};
 }
 
 // One ray per lane (active: the lane has one).  sc is uniform.
@@ -227,8 +223,20 @@ __device__ __forceinline__ TravOut scan_ray(const DevScene& sc, f3 o, f3 d, floa
     });
     TravOut r{kMiss, tmax, false};
     if (!active) return r;
-    if (any) r.hit = scan_end_any(sc, o, d, tmax, eps, err, n) || scan_plane_stops(sc, o, d, tmax, eps);
-    else r = scan_end_closest(sc, o, d, tmax, eps, err, n);
+    if (any) {
+        r.hit = scan_end_any(sc, o, d, tmax, eps, err, n);
+        if (r.hit) return r;
+    } else {
+        scan_end_closest(sc, o, d, tmax, eps, err, n, r.t, r.prim);
+    }
+    n.clear();
+    scan_planes(sc, o, d, eps, n);
+    if (any) {
+        r.hit = scan_plane_stops(sc, o, d, tmax, eps, n);
+    } else {
+        scan_plane_hits(sc, o, d, eps, n, r.t, r.prim);
+        r.hit = r.prim != kMiss;
+    }
     return r;
 }
 
@@ -276,10 +284,100 @@ __device__ __forceinline__ TravOut scan_pair(const DevScene& sc, f3 o, bool sh, 
         n.add(SphereTerms(oc, cc, d).near(), lo, (1u << 30) | i);
         m.add(SphereTerms(oc, cc, sd).near(), lo, i);
     });
-    occluded = false;
-    if (sh) occluded = scan_end_any(sc, o, sd, st, eps, err, m) || scan_plane_stops(sc, o, sd, st, eps);
-    if (!seg) return TravOut{kMiss, tmax, false};
-    return scan_end_closest(sc, o, d, tmax, eps, err, n);
+    occluded = sh && scan_end_any(sc, o, sd, st, eps, err, m);
+    TravOut r{kMiss, tmax, false};
+    if (seg) scan_end_closest(sc, o, d, tmax, eps, err, n, r.t, r.prim);
+    n.clear();
+    m.clear();
+    scan_planes(sc, o, d, eps, n);
+    if (sh && !occluded) {
+        scan_planes(sc, o, sd, eps, m);
+        occluded = scan_plane_stops(sc, o, sd, st, eps, m);
+    }
+    if (seg) scan_plane_hits(sc, o, d, eps, n, r.t, r.prim);
+    r.hit = r.prim != kMiss;
+    return r;
+}
+
+// scan_pair by four lanes: lane 4k has the rays (sh, seg; its three neighbours
+// none), each of the four tests every fourth primitive for them, and two
+// exchanges bring the least two together.  For images so small that lanes are
+// idle anyway and the time is a pixel's serial chain, of which the tests of 33
+// spheres are a third (256^2, 16 spp, 33 spheres, forward + backward
+// 1134 -> 1032 us; 64^2 reference scene 90.5 -> 84.7).
+__device__ __forceinline__ float quad_first(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x00, 0xF, 0xF, true));
+}
+__device__ __forceinline__ f3 quad_first(f3 v) { return f3{quad_first(v.x), quad_first(v.y), quad_first(v.z)}; }
+template <int PERM>
+__device__ __forceinline__ void quad_merge(Nearest& n)
+{
+    const float b = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(n.best), PERM, 0xF, 0xF, true));
+    const float s = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(n.second), PERM, 0xF, 0xF, true));
+    const uint32_t k = (uint32_t)__builtin_amdgcn_mov_dpp((int)n.key, PERM, 0xF, 0xF, true);
+    n.second = fminf(fmaxf(n.best, b), fminf(n.second, s));
+    n.key = b < n.best ? k : n.key;
+    n.best = fminf(n.best, b);
+}
+__device__ __forceinline__ void quad_merge(Nearest& n)
+{
+    quad_merge<0xB1>(n);   // lanes 1 0 3 2
+    quad_merge<0x4E>(n);   // lanes 2 3 0 1
+}
+// Calls body(row, i) for this lane's quarter of the rows.
+template <class Body>
+__device__ __forceinline__ void for_quad_rows(const float4* rows, uint32_t n, uint32_t q, Body&& body)
+{
+    float4 a = rows[q];
+    for (uint32_t i = 0; i < n; i += kScanRun) {
+        const float4 a1 = rows[i + kScanRun + q];
+        body(a, i + q);
+        a = a1;
+    }
+}
+__device__ __forceinline__ TravOut scan_pair_quad(const DevScene& sc, f3 o, bool sh, f3 sd, float st, bool seg, f3 d,
+                                                  float tmax, float eps, bool& occluded)
+{
+    const uint32_t q = __lane_id() & 3u;
+    const f3 qo = quad_first(o), qd = quad_first(d), qs = quad_first(sd);
+    const float err = scan_error(sc, qo), lo = eps - err;
+    Nearest n, m, np, mp;
+    n.clear();
+    m.clear();
+    np.clear();
+    mp.clear();
+    for (uint32_t i = q; i < sc.n_tris; i += 4u) {
+        const float4* p = reinterpret_cast<const float4*>(sc.scan_tris + i);
+        const float4 a = p[0], b = p[1], c = p[2];
+        const f3 v0{a.x, a.y, a.z}, e1{b.x, b.y, b.z}, e2{c.x, c.y, c.z};
+        n.add(tri_t(qo, qd, v0, e1, e2, eps), eps, i);
+        m.add(tri_t(qo, qs, v0, e1, e2, eps), eps, i);
+    }
+    for_quad_rows(sc.scan_sph, sc.n_spheres, q, [&](float4 s, uint32_t i) __attribute__((always_inline)) {
+        const f3 oc = sub(qo, f3{s.x, s.y, s.z});
+        const float cc = dot(oc, oc) - s.w;
+        n.add(SphereTerms(oc, cc, qd).near(), lo, (1u << 30) | i);
+        m.add(SphereTerms(oc, cc, qs).near(), lo, i);
+    });
+    const float lop = eps * (1.0f - 0x1p-18f);
+    for_quad_rows(sc.scan_planes, sc.n_planes, q, [&](float4 p, uint32_t i) __attribute__((always_inline)) {
+        const f3 N{p.x, p.y, p.z};
+        const float num = p.w + dot(qo, N);
+        np.add(-num * __builtin_amdgcn_rcpf(dot(qd, N)), lop, i);
+        mp.add(-num * __builtin_amdgcn_rcpf(dot(qs, N)), lop, i);
+    });
+    quad_merge(n);
+    quad_merge(m);
+    quad_merge(np);
+    quad_merge(mp);
+    occluded = sh && (scan_end_any(sc, o, sd, st, eps, err, m) || scan_plane_stops(sc, o, sd, st, eps, mp));
+    TravOut r{kMiss, tmax, false};
+    if (!seg) return r;
+    scan_end_closest(sc, o, d, tmax, eps, err, n, r.t, r.prim);
+    scan_plane_hits(sc, o, d, eps, np, r.t, r.prim);
+    r.hit = r.prim != kMiss;
+    return r;
 }
 
 }  // namespace vkr

@@ -113,7 +113,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
     // Lane state.
     bool has = false;
     ItemPool pool;
-    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + (wbase >> 6), gridDim.x * (BLOCK / 64), A.width);
+    pool.start((uint32_t)blockIdx.x * (BLOCK / 64) + (wbase >> 6), gridDim.x * (BLOCK / 64), A.width, SCAN && !POOL && !BATCH && A.width <= kQuadWidth);
     uint32_t job = 0, px = 0, py = 0;
     float uvx = 0.0f, uvy = 0.0f, salt = 0.0f;
     uint32_t smp = 0, depth = 0;
@@ -304,7 +304,11 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
             bool occluded = false;
             for_each_job<BATCH>(A, job_at, job, has, [&](const JobDesc& jt, bool mine) __attribute__((always_inline)) {
                 if (!mine) return;
-                if constexpr (SCAN)
+                if constexpr (SCAN && !BATCH)
+                    tr = A.width <= kQuadWidth
+                             ? scan_pair_quad(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, occluded)
+                             : scan_pair(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, occluded);
+                else if constexpr (SCAN)
                     tr = scan_pair(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, occluded);
                 else
                     tr = traverse_pair<BLOCK, COUNT>(jt.sc, ro, sh, sd, st, has && seg, rd, tmax, jt.eps, stk, wc,

@@ -514,8 +514,8 @@ __device__ __forceinline__ DevCounters* counter_bank(const CounterRef& c, uint32
     return c.banks + (block & c.mask);
 }
 
-// A wave's view of a launch's pool of work items, which its lanes 0 .. width - 1
-// take.  The wave starts with the `width` items of its own number; the pool's
+// A wave's view of a launch's pool of work items, which `width` of its lanes
+// take: lanes 0 .. width - 1, or with quads every fourth lane.  The wave starts with the `width` items of its own number; the pool's
 // cursor counts from the last wave's up, so the waves of a launch do not open
 // it with a queue of atomics on one address (11.5 ns each).  Later claims take just the idle lanes' items: a
 // wave that kept a run of items to itself (a share of what is left, up to 64)
@@ -526,12 +526,15 @@ struct ItemPool {
     uint32_t own;             // first of the wave's own items (kNoItem: taken)
     uint32_t shared;          // items below are the waves' own
     uint32_t width;           // lanes that take items
+    unsigned long long takers;   // which ones
     bool dry;                 // nothing is left behind the cursor
     static constexpr uint32_t kNoItem = 0xFFFFFFFFu;
 
-    __device__ __forceinline__ void start(uint32_t wave, uint32_t waves, uint32_t width_)
+    __device__ __forceinline__ void start(uint32_t wave, uint32_t waves, uint32_t width_, bool quads = false)
     {
         width = width_;
+        const uint32_t span = quads ? 4u * width : width;
+        takers = (span >= 64u ? ~0ull : (1ull << span) - 1ull) & (quads ? 0x1111111111111111ull : ~0ull);
         own = wave * width;
         shared = waves * width;
         dry = false;
@@ -541,7 +544,7 @@ struct ItemPool {
     template <class Claim>
     __device__ __forceinline__ void refill(uint32_t* cursor, uint32_t total, uint32_t chunk, bool has, Claim&& claim)
     {
-        const unsigned long long need = __ballot(!has && __lane_id() < width);
+        const unsigned long long need = __ballot(!has) & takers;
         const uint32_t n = (uint32_t)__popcll(need);
         if (n == 0u || n < min(chunk, width) || dry) return;
         uint32_t base = own;

@@ -185,7 +185,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(const AdjointLaunch A)
             if (type == VKR_MAT_DIFFUSE) {
                 const float r2 = rng_next(salt, uvx, uvy);
                 const float phi = kTwoPi * rng_next(salt, uvx, uvy);
-                const f3 dj = muls(jitter(N, phi, sqrtf(r2), sqrtf(1.0f - r2)), 1.0f - m->metalness);
+                const f3 dj = muls(jitter(N, phi, sqrt_rn(r2), sqrt_rn(1.0f - r2)), 1.0f - m->metalness);
                 hm = m;
                 e = f3{0.0f, 0.0f, 0.0f};
                 ei = 0;
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint(const AdjointLaunch A)
             if (hs != kMiss && nchain < kMaxAdjDepth) chain[(nchain++) * BLOCK] = hs;
             cstar = argmax3(mask);
             if (!term) {
-                mask = muls(mask, 1.0f / max3(mask));
+                mask = muls(mask, recip_rn(max3(mask)));
                 ++depth;
             }
         }

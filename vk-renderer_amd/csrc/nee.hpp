@@ -159,10 +159,10 @@ __device__ __forceinline__ NeeEval nee_eval(const NeeHit& h, const vkr_sphere* S
     float dist;
     const f3 w0 = normalize_len(l0, dist);
     q.tl = dist - sr;
-    const float cos_a_max = sqrtf(1.0f - gclamp(sr * sr / dot(l0, l0), 0.0f, 1.0f));
+    const float cos_a_max = sqrt_rn(1.0f - gclamp(sr * sr / dot(l0, l0), 0.0f, 1.0f));
     const float cosa = gmix(cos_a_max, 1.0f, rng_next(salt, uvx, uvy));
     const float phi = kTwoPi * rng_next(salt, uvx, uvy);
-    q.L = jitter_w(w0, phi, sqrtf(1.0f - cosa * cosa), cosa);
+    q.L = jitter_w(w0, phi, sqrt_rn(1.0f - cosa * cosa), cosa);
 
     const float x = q.tl / sr + 1.0f;
     q.x2 = x * x;

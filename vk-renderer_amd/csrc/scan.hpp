@@ -87,7 +87,7 @@ struct SphereTerms {
         h = dt * dt - cc;
     }
     __device__ __forceinline__ float near() const { return -dt - __builtin_amdgcn_sqrtf(h); }   // NaN when h < 0
-    __device__ __forceinline__ float exact() const { return h < 0.0f ? -1.0f : -dt - sqrtf(h); }
+    __device__ __forceinline__ float exact() const { return h < 0.0f ? -1.0f : -dt - sqrt_rn(h); }
 };
 
 // The reference's loop over triangles and spheres.  any: stops at the first

@@ -430,7 +430,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
             acc = add(acc, mul(mask, add(em, e)));
             mask = mul(mask, ld3(hm->albedo));
             if (!term) {
-                mask = muls(mask, 1.0f / max3(mask));
+                mask = muls(mask, recip_rn(max3(mask)));
                 ++depth;
             }
             path_end = !seg;
@@ -538,7 +538,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
             if (type == VKR_MAT_DIFFUSE) {                           // :451-513
                 const float r2 = rng_next(salt, uvx, uvy);
                 const float phi = kTwoPi * rng_next(salt, uvx, uvy);
-                const f3 dj = muls(jitter(N, phi, sqrtf(r2), sqrtf(1.0f - r2)), 1.0f - m->metalness);
+                const f3 dj = muls(jitter(N, phi, sqrt_rn(r2), sqrt_rn(1.0f - r2)), 1.0f - m->metalness);
                 hm = m;
                 ei = 0;
                 e = f3{0.0f, 0.0f, 0.0f};
@@ -567,7 +567,7 @@ __device__ __forceinline__ void path_program(const PathLaunch& A)
                 }
                 // (a type outside the switch goes straight on to the roulette)
                 if (!roulette(j, mask)) {
-                    mask = muls(mask, 1.0f / max3(mask));
+                    mask = muls(mask, recip_rn(max3(mask)));
                     ++depth;
                     seg = depth < j.max_depth;
                     if (seg) {

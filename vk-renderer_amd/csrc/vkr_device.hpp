@@ -76,7 +76,29 @@ __device__ __forceinline__ f3 cross(f3 a, f3 b)
 {
     return f3{a.y * b.z - b.y * a.z, a.z * b.x - b.z * a.x, a.x * b.y - b.x * a.y};
 }
-__device__ __forceinline__ float length(f3 a) { return sqrtf(dot(a, a)); }
+// 1 / x and sqrt(x), rounded to nearest as the division and sqrtf round: one
+// Newton step from the hardware's estimate gives their bits for every float of
+// [2^-64, 2^64) (all 2^30 of them compared).  21 and 31 cycles of a SIMD with
+// an addition, against 48 and 60.  (Out of line for the rest: in line it costs
+// the path kernels 30 registers.)  1024^2 Whitted frame 50.7 -> 46.6 us, 65
+// spheres 512^2 374 -> 370.
+__device__ __forceinline__ bool mid_range(float x) { return __float_as_uint(x) - (63u << 23) < (128u << 23); }
+__device__ __attribute__((noinline)) float recip_long(float x) { return 1.0f / x; }
+__device__ __attribute__((noinline)) float sqrt_long(float x) { return sqrtf(x); }
+__device__ __forceinline__ float recip_rn(float x)
+{
+    if (__builtin_expect(!mid_range(x), 0)) return recip_long(x);
+    const float y = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float sqrt_rn(float x)
+{
+    if (__builtin_expect(!mid_range(x), 0)) return sqrt_long(x);
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+__device__ __forceinline__ float length(f3 a) { return sqrt_rn(dot(a, a)); }
 // v / length(v), and the length: the root as two steps of g += (x - g^2) / (2
 // sqrt x) in double, whose error (2^-53) is below the least distance of a
 // float's root from a midpoint (2^-51), then the quotients as in divs with
@@ -120,7 +142,7 @@ __device__ __forceinline__ f3 refract(f3 I, f3 N, float eta)
     const float d = dot(N, I);
     const float k = 1.0f - eta * eta * (1.0f - d * d);
     if (k < 0.0f) return f3{0.0f, 0.0f, 0.0f};
-    return sub(muls(I, eta), muls(N, eta * d + sqrtf(k)));
+    return sub(muls(I, eta), muls(N, eta * d + sqrt_rn(k)));
 }
 __device__ __forceinline__ float max3(f3 e) { return gmax(gmax(e.x, e.y), e.z); }
 
@@ -434,7 +456,7 @@ __device__ __forceinline__ float sphere_t(f3 o, f3 d, f3 c, float r)
     const float cc = dot(oc, oc) - r * r;
     const float h = b * b - 4.0f * cc;
     if (h < 0.0f) return -1.0f;
-    return (-b - sqrtf(h)) / 2.0f;
+    return (-b - sqrt_rn(h)) / 2.0f;
 }
 __device__ __forceinline__ float plane_t(f3 o, f3 d, f3 N, float len)
 {
@@ -449,7 +471,7 @@ __device__ __forceinline__ float tri_t(f3 o, f3 d, f3 v0, f3 e1, f3 e2, float ep
     const f3 pvec = cross(d, e2);
     const float det = dot(e1, pvec);
     if (det < eps) return -1.0f;
-    const float inv = 1.0f / det;
+    const float inv = recip_rn(det);
     const f3 tvec = sub(o, v0);
     const float u = dot(tvec, pvec) * inv;
     if (u < 0.0f || u > 1.0f) return -1.0f;

@@ -53,8 +53,9 @@ constexpr uint32_t kMaxLeaf = 8;
 constexpr uint32_t kDefaultLeaf = 2;
 inline uint32_t default_leaf(uint32_t n_emitters) { return n_emitters >= 2u ? 1u : kDefaultLeaf; }
 // Default depth cap: trees of at most 23 levels run the path kernel with a
-// 24-entry stack (one entry holds the end marker), which keeps 5 waves per
-// SIMD resident instead of 4.  The SAH split search respects the cap.
+// 24-entry stack (one entry holds the end marker), which keeps 5 waves of the
+// pooled kernel resident per SIMD instead of 4.  The SAH split search respects
+// the cap.
 constexpr uint32_t kDefaultMaxDepth = 23;
 
 struct alignas(16) BvhNode {

@@ -19,16 +19,22 @@ namespace vkr {
 
 constexpr uint32_t kDone = 0xFFFFFFFFu;
 
-
 // A wave leaves the node loop for the leaf pass once at least kLeafExit8/8
 // of its lanes that are still traversing wait at a leaf (or, in the pooled
 // loop, for a new ray); the others keep their place in the tree and go on in
-// the next round.  Every ray still visits the same nodes and primitives in
-// the same order (results do not depend on it); only the grouping of lanes
-// into wave iterations changes.  4/8 measured best on incoherent 1080p /
-// 100k-triangle frames with leaves of at most 2 primitives (2/8 and 6/8 are
-// 12% and 4% slower with the pooled loop).
-constexpr uint32_t kLeafExit8 = 4;
+// the next round (results do not depend on it; only the grouping of lanes
+// into wave iterations changes).  With one ray a lane 4/8 measured best (3/8
+// and 5/8 up to 3% slower on the 1080p heightfield).
+//
+// In the pooled loop a lane that reaches a leaf keeps it for later and goes on
+// with its next node; it waits at a second leaf, or when nothing else is left.
+// That fills the node steps, which are most of the time, for a few nodes that
+// the leaf's hit would have spared: with 3/8 the 1080p frame of the
+// 100k-triangle soup takes 72.8 -> 71.2 ms, 1M triangles 853x477 13.1 -> 12.8,
+// 5k triangles 512^2 4.43 -> 4.19 (2/8 the same, 5/8 4% slower).  With one ray
+// a lane it loses 3%: closest hits cull more than shadow rays.  The counting
+// kernel tests each leaf at once, so its counts stay the tree's own.
+constexpr uint32_t kLeafExit8 = 4, kLeafExit8Pool = 3;
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
@@ -82,6 +88,7 @@ struct Ray {
     float ct0, ct1, ct2, ct3;
     uint32_t ck0, ck1, ck2, ck3;
     bool any, ovf, occluded, nan_ray;
+    uint32_t post;  // a leaf that is passed but not tested yet, or kDone (pooled loop)
     uint32_t ref;   // >= 0 (as int): inner node; < -1: leaf; kDone: traversal over
     int sp;         // stack entries; entry 0 is always kDone, so a pop needs no bounds check
 
@@ -132,6 +139,7 @@ struct Ray {
         pad = q * __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(__builtin_fmaf(sc.sph_rmin, sc.sph_rmin, q)) + sc.sph_rmin);
         pad = pad < 3e38f ? pad : 3e38f;   // (also from 0 / 0 and inf / inf)
         ref = (sc.has_bvh && !nan_ray) ? 0u : kDone;
+        post = kDone;
         sp = 1;   // above the kDone entry the traversal loops keep at the bottom
     }
 
@@ -184,19 +192,36 @@ struct Ray {
         sp += (h0 && h1 ? 1 : 0) - (none ? 1 : 0);
     }
 
-    // Tests the primitives of leaf `ref`, then pops the stack.
-    template <int BLOCK, bool COUNT>
-    __device__ __forceinline__ void leaf(const TreePtrs& sc, float eps, uint32_t* stk, WorkCnt& wc)
+    template <int BLOCK>
+    __device__ __forceinline__ void pop(uint32_t* stk)
+    {
+        ref = stk[(sp - 1) * BLOCK];   // the bottom entry is kDone
+        --sp;
+    }
+    // Keeps leaf `ref` for later and pops the stack, if none is kept.
+    template <int BLOCK>
+    __device__ __forceinline__ void postpone(uint32_t* stk)
+    {
+        if ((int)ref < -1 && post == kDone) {
+            post = ref;
+            pop<BLOCK>(stk);
+        }
+    }
+    __device__ __forceinline__ bool over() const { return ref == kDone && post == kDone; }
+
+    // Tests the primitives of leaf `at`.
+    template <bool COUNT>
+    __device__ __forceinline__ void leaf(const TreePtrs& sc, uint32_t at, float eps, WorkCnt& wc)
     {
         const float inf = __builtin_huge_valf();
         const float win = 4.0f * eps;
         if (COUNT) count_wave(wc.wave_leaves);
-        const uint32_t count = ((ref >> kRefCountShift) & 7u) + 1u;
-        const uint32_t first = ref & kRefFirstMask;
+        const uint32_t count = ((at >> kRefCountShift) & 7u) + 1u;
+        const uint32_t first = at & kRefFirstMask;
         for (uint32_t i = 0; i < count; ++i) {
             float t;
             uint32_t key;
-            if (ref & kRefSphere) {
+            if (at & kRefSphere) {
                 const float4 s4 = sc.sph[first + i];
                 if (COUNT) wc.spheres++;
                 t = sphere_t(o, d, f3{s4.x, s4.y, s4.z}, s4.w);
@@ -247,12 +272,25 @@ struct Ray {
                 set_cull(fminf(tmin, tmax_eps) + win);
             }
         }
-        if (occluded) {
-            ref = kDone;
-        } else {
-            ref = stk[(sp - 1) * BLOCK];   // the bottom entry is kDone
-            --sp;
-        }
+    }
+
+    // Tests leaf `ref`, then pops the stack.
+    template <int BLOCK, bool COUNT>
+    __device__ __forceinline__ void leaf_now(const TreePtrs& sc, float eps, uint32_t* stk, WorkCnt& wc)
+    {
+        leaf<COUNT>(sc, ref, eps, wc);
+        if (occluded) ref = kDone;
+        else pop<BLOCK>(stk);
+    }
+    // Tests the leaf that was kept; one that waits at `ref` takes its place.
+    template <int BLOCK, bool COUNT>
+    __device__ __forceinline__ void leaf_kept(const TreePtrs& sc, float eps, uint32_t* stk, WorkCnt& wc)
+    {
+        const uint32_t at = post;
+        post = kDone;
+        leaf<COUNT>(sc, at, eps, wc);
+        if (occluded) ref = kDone;
+        else postpone<BLOCK>(stk);
     }
 
     // After traversal: the planes (a linear list) and, for closest-hit rays,
@@ -321,9 +359,9 @@ struct Ray {
 // (at a leaf, or for a new ray).  Both loops take two node steps per test
 // (the test's ballots cost about as much as a third of a step): 3-5% faster
 // on 1080p frames of the 100k-triangle soup and the 2M-triangle heightfield.
-__device__ __forceinline__ bool leave_nodes(uint32_t nn, uint32_t nw)
+__device__ __forceinline__ bool leave_nodes(uint32_t nn, uint32_t nw, uint32_t exit8)
 {
-    return nn == 0 || (nw > 0 && nw * 8u >= (nw + nn) * kLeafExit8);
+    return nn == 0 || (nw > 0 && nw * 8u >= (nw + nn) * exit8);
 }
 
 // Whether a plane stops a shadow ray (the tests of Ray::finish; their order
@@ -367,12 +405,12 @@ __device__ __forceinline__ TravOut traverse_pair(const DevScene& sc, f3 o, bool 
         while (true) {
             const uint32_t nn = (uint32_t)__popcll(__ballot((int)r.ref >= 0));
             const uint32_t nw = (uint32_t)__popcll(__ballot((int)r.ref < -1 || (next && r.ref == kDone)));
-            if (leave_nodes(nn, nw)) break;
+            if (leave_nodes(nn, nw, kLeafExit8)) break;
             if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
             if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
         }
         if (__ballot(r.ref != kDone || next) == 0) break;
-        if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(tree, eps, stk, wc);
+        if ((int)r.ref < -1) r.leaf_now<BLOCK, COUNT>(tree, eps, stk, wc);
     }
     if (r.any) occluded = r.occluded;   // a shadow ray with no segment behind it
     if (!seg) return TravOut{kMiss, tmax, false};
@@ -451,6 +489,7 @@ __device__ __forceinline__ void traverse_pool(const JobDesc& j, uint32_t total, 
     const float eps = j.eps;
     Ray r;
     r.ref = kDone;
+    r.post = kDone;
     stk[0] = kDone;
     uint32_t cur = kNone;
     uint32_t next = 0;   // wave-uniform pool cursor
@@ -458,7 +497,7 @@ __device__ __forceinline__ void traverse_pool(const JobDesc& j, uint32_t total, 
         // Post finished rays and hand out new ones until every lane is busy
         // or the pool is empty.
         while (true) {
-            if (cur != kNone && r.ref == kDone) {
+            if (cur != kNone && r.over()) {
                 const TravOut t = r.finish<COUNT>(j.sc, eps, wc);
                 const uint32_t owner = cur >> 5;
                 if (r.any) {
@@ -481,18 +520,23 @@ __device__ __forceinline__ void traverse_pool(const JobDesc& j, uint32_t total, 
                 }
                 next += (uint32_t)__popcll(want);
             }
-            if (__ballot(cur != kNone && r.ref == kDone) == 0) break;
+            if (__ballot(cur != kNone && r.over()) == 0) break;
         }
         if (__ballot(cur != kNone) == 0) break;
         const bool more = next < total;
         while (true) {
             const uint32_t nn = (uint32_t)__popcll(__ballot((int)r.ref >= 0));
-            const uint32_t nw = (uint32_t)__popcll(__ballot((int)r.ref < -1 || (more && r.ref == kDone)));
-            if (leave_nodes(nn, nw)) break;
+            const uint32_t nw = (uint32_t)__popcll(__ballot((int)r.ref < -1 || (r.ref == kDone && (more || r.post != kDone))));
+            if (leave_nodes(nn, nw, COUNT ? kLeafExit8 : kLeafExit8Pool)) break;
             if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
             if ((int)r.ref >= 0) r.node<BLOCK, COUNT>(tree.nodes, stk, wc);
+            if constexpr (!COUNT) r.postpone<BLOCK>(stk);
         }
-        if ((int)r.ref < -1) r.leaf<BLOCK, COUNT>(tree, eps, stk, wc);
+        if constexpr (COUNT) {
+            if ((int)r.ref < -1) r.leaf_now<BLOCK, COUNT>(tree, eps, stk, wc);
+        } else {
+            if (r.post != kDone) r.leaf_kept<BLOCK, COUNT>(tree, eps, stk, wc);
+        }
     }
 }
 
@@ -515,8 +559,8 @@ __device__ __forceinline__ DevCounters* counter_bank(const CounterRef& c, uint32
 }
 
 // A wave's view of a launch's pool of work items, which `width` of its lanes
-// take: lanes 0 .. width - 1, or with quads every fourth lane.  The wave starts with the `width` items of its own number; the pool's
-// cursor counts from the last wave's up, so the waves of a launch do not open
+// take: lanes 0 .. width - 1, or with quads every fourth lane.  The wave starts
+// with the `width` items of its own number; the pool's cursor counts from the last wave's up, so the waves of a launch do not open
 // it with a queue of atomics on one address (11.5 ns each).  Later claims take just the idle lanes' items: a
 // wave that kept a run of items to itself (a share of what is left, up to 64)
 // made fewer claims but left waves idle at the end of the launch while others

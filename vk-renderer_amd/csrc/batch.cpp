@@ -73,7 +73,7 @@ PathLaunch batch_launch(const BatchPlan& plan, const JobDesc* djobs, const uint3
     a.n_jobs = n;
     a.total = (uint32_t)plan.total;
     a.persistent = 1u;
-    a.chunk = chunk ? chunk : kDefaultChunk;
+    a.chunk = chunk;
     a.pool = pool;
     a.counters = cnt;
     return a;
@@ -122,6 +122,17 @@ uint64_t batch_key(const vkr_scene_job* jobs, uint32_t n)
     return h;
 }
 
+// The refill threshold of a batch whose caller and autotuner gave none.
+uint32_t batch_chunk(const BatchPlan& plan)
+{
+    uint32_t spp = 0, depth = 0;
+    for (const JobDesc& j : plan.jobs) {
+        spp = std::max(spp, j.spp);
+        depth = std::max(depth, j.max_depth);
+    }
+    return default_chunk(batch_variant(plan, 128u, false), spp, depth);
+}
+
 struct BatchShape {
     uint32_t block, chunk;
 };
@@ -150,7 +161,7 @@ BatchShape batch_shape(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n, Batc
         }
     }
     if (!s.block) s.block = 128u;
-    if (!s.chunk) s.chunk = kDefaultChunk;
+    if (!s.chunk) s.chunk = batch_chunk(plan);
     if (!tuned && plan.stack == 24u && plan.tree_depth <= 8u) {
         const PathVariant v4{s.block, 32u, false, plan.jobs.size() > 1u, plan.pool};
         const uint64_t resident4 = (uint64_t)persistent_grid(v4, ctx->device) * s.block;
@@ -362,7 +373,7 @@ vkr_error vkr_autotune(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd, c
         p.chunk = c.chunk;
         p.sched = c.sched;
         // The stack variant is chosen through a temporary tuning entry.
-        ctx->tuned.push_back(TuneEntry{scene, p.width, p.height, c.block, c.chunk ? c.chunk : kDefaultChunk, c.stack, c.sched});
+        ctx->tuned.push_back(TuneEntry{scene, p.width, p.height, c.block, c.chunk, c.stack, c.sched});
         float total = 0.0f;
         vkr_error e = vkr_trace_frame(ctx, scene, fd, &p, outputs, nullptr);
         for (uint32_t r = 0; r < repeats && e == VKR_SUCCESS; ++r) {
@@ -387,7 +398,7 @@ vkr_error vkr_autotune(vkr_ctx* ctx, uint32_t scene, const vkr_frame_data* fd, c
             win = c;
         }
     }
-    ctx->tuned.push_back(TuneEntry{scene, params->width, params->height, win.block, win.chunk ? win.chunk : kDefaultChunk,
+    ctx->tuned.push_back(TuneEntry{scene, params->width, params->height, win.block, win.chunk,
                                    win.stack, win.sched});
     out->block = win.block;
     out->chunk = win.chunk;
@@ -441,7 +452,7 @@ vkr_error vkr_autotune_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n
     // Coordinate descent (one batch launch is long, a full grid is not
     // affordable): workgroup size at the default chunk, then the pool chunk,
     // then the stack depth.  One warm launch loads the kernels first.
-    uint32_t best_b = 128u, best_c = kDefaultChunk, best_s = needed;
+    uint32_t best_b = 128u, best_c = batch_chunk(plan), best_s = needed;
     float best = 3.4e38f, ms = 0.0f;
     vkr_error e = vkr_trace_batch(ctx, jobs, n_jobs, best_b, best_c, nullptr);
     if (e != VKR_SUCCESS) return e;
@@ -449,7 +460,9 @@ vkr_error vkr_autotune_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n
         if ((e = time_shape(b, best_c, best_s, ms)) != VKR_SUCCESS) return e;
         if (ms < best) { best = ms; best_b = b; }
     }
-    for (uint32_t c : {1u, 4u, 16u, 32u}) {
+    const uint32_t default_c = best_c;
+    for (uint32_t c : {1u, 4u, 8u, 16u, 32u, 64u}) {
+        if (c == default_c) continue;
         if ((e = time_shape(best_b, c, best_s, ms)) != VKR_SUCCESS) return e;
         if (ms < best) { best = ms; best_c = c; }
     }

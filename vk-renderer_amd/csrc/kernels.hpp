@@ -106,10 +106,6 @@ struct CounterRef {
     uint32_t mask;                // number of banks - 1
 };
 
-// Default pool refill threshold: a wave claims new pixels once at least this
-// many of its lanes are idle (8-16 measured best at 1080p; 32 idles lanes,
-// 1 refills too often).
-constexpr uint32_t kDefaultChunk = 8u;
 
 // Most work items one launch's 32-bit pool cursor hands out.  A resident
 // wave can add up to 64 to the cursor after the last item has gone (its one
@@ -196,6 +192,26 @@ struct PathVariant {
     bool count, batch, pool;
     bool scan = false;   // every job's scene is scanned: no tree, no stack (stack is ignored)
 };
+
+// Default pool refill threshold: a wave claims new pixels once at least this
+// many of its lanes are idle.  A claim is an atomic on one address, 11.5 ns
+// after the one before it, and takes all waves' turn; lanes idle meanwhile.
+// Against 8 (one MI355X):
+//   one frame of a tree or with the ray pool: 1 to 32 within 2%, 48 and 64 3-15%
+//   slower (1080p heightfield, 100k-triangle soup), so 8;
+//   one ray a lane over a scanned scene costs so little a pixel that the claims
+//   bound it: 64 takes the 1024^2 reference scene, 4 spp, from 1115 to 854 us
+//   (16: 867, 32: 942), 1 spp 428 to 233, 33 spheres 720p 404 to 363.  That
+//   ends where spp times bounces reaches 32 (1024x768 reference scene 8 spp, 4
+//   bounces 1232 / 1228 us, 6 spp, 8 bounces 1140 / 1146, 8 spp, 8 bounces
+//   1355 / 1422);
+//   batches, whose jobs' pixels differ more: 32 takes 64 mixed scenes from 1482
+//   to 1352 ms, eight soups 265 to 255, two heightfields 1809 to 1795 us.
+inline uint32_t default_chunk(const PathVariant& v, uint32_t spp, uint32_t max_depth)
+{
+    if (v.scan && !v.pool && (uint64_t)spp * max_depth <= 32u) return 64u;
+    return v.batch ? 32u : 8u;
+}
 
 hipError_t launch_path(const PathLaunch& a, const PathVariant& v, uint32_t grid, hipStream_t s);
 hipError_t launch_whitted(const JobDesc& j, CounterRef c, hipStream_t s);

@@ -263,8 +263,8 @@ enum {
     /* vkr_trace_frame only (path kernel, max_depth <= 10, no decision
      * flags): also keeps, in the context, what the first pass of vkr_adjoint
      * computes for this frame (each sample's random-stream position at its
-     * start and which channels of its clamp saturate, 8 bytes per sample;
-     * growing that buffer waits for the device).  The next
+     * start and which channels of its clamp saturate, 8 bytes per sample,
+     * and each pixel's primary hit, 8 bytes per pixel; growing that buffer waits for the device).  The next
      * vkr_adjoint with the same scene, sphere parameters, frame data and
      * trace parameters then runs only its second pass.  The image is
      * unchanged.  Refused by vkr_trace_batch, vkr_batch_graph_create and
@@ -371,7 +371,7 @@ vkr_error vkr_autotune_batch(vkr_ctx* ctx, const vkr_scene_job* jobs, uint32_t n
  * accumulates dLoss/dparams into d_params (device, 7 * n_spheres + 1 floats,
  * layout of vkr_scene_set_sphere_params; the caller zeroes it).  Paths are
  * recomputed from the RNG stream, not stored: a first pass keeps 8 bytes per
- * (pixel, sample) in a context buffer (grown on demand, which waits for the
+ * (pixel, sample) and 8 per pixel in a context buffer (grown on demand, which waits for the
  * device) so that the second replays every sample in its own lane.  The
  * first pass is skipped when the buffer already holds its records for the
  * same scene, sphere parameters, frame data and trace parameters (width,
@@ -419,7 +419,8 @@ typedef struct vkr_counters {
     uint64_t window_overflow; /* closest-hit tie window exceeded (documented near-ties) */
     uint64_t rays_traced;     /* rays actually traversed: shadow rays whose contribution is
                                  exactly 0 whatever their outcome are counted in `rays`
-                                 but not traversed */
+                                 but not traversed, and the primary ray that a
+                                 pixel's samples share is traversed once */
     uint64_t wave_node_iters; /* wave-level BVH node-loop iterations (VKR_CTX_COUNT_WORK);
                                  SIMD efficiency = nodes_visited / (64 * wave_node_iters) */
     uint64_t wave_leaf_iters; /* wave-level leaf visits (VKR_CTX_COUNT_WORK) */

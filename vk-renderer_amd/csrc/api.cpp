@@ -437,28 +437,25 @@ static vkr_error ensure_adj_records(vkr_ctx* ctx, JobDesc& j)
     return VKR_SUCCESS;
 }
 
-// Trees of depth <= 23 can take the 24-entry-stack kernel, which keeps 5
-// waves per SIMD resident (4 with the 32-entry stack, 2 to 3 with the
-// 64-entry one, both with more registers and fewer spills).  Untuned
-// launches choose by the tree's depth and, with single rays, by the image
-// size against the lanes the 4-wave kernel keeps resident (one MI355X):
-// - trees deeper than 8 levels, where node fetches dominate: the pooled
-//   kernel takes the fifth wave at any size, as narrow waves fill the grid
-//   (256^2 frame of a 50k-triangle soup 7.4 against 8.6 ms); with single rays
-//   it pays off only with well over twice the resident pixels;
+// Trees of depth <= 23 can take the 24-entry-stack kernel, which keeps 5 waves
+// of the pooled kernel per SIMD resident (4 with the 32-entry stack, 2 to 3
+// with the 64-entry one, both with more registers and fewer spills).  Untuned
+// launches choose by the tree's depth (one MI355X):
+// - trees deeper than 8 levels, where node fetches dominate: the 24-entry kernel
+//   (pooled, 256^2 frame of a 50k-triangle soup 7.4 against 8.6 ms; with single
+//   rays, 4 waves either way, within 1%);
 // - shallow trees, where shading dominates: the 32-entry kernel (160 spheres,
 //   a quarter lights, 256^2: 0.74 against 0.78 ms with 24 entries, 0.85 with
-//   64), or for single rays the 64-entry one when the grid holds every pixel
-//   at once.
+//   64), or for single rays the 64-entry one when the 32-entry kernel's grid
+//   holds every pixel at once (181 spheres, 64x48: 132 against 142 us with 24).
 static uint32_t default_stack(const PathVariant& v, uint32_t total, uint32_t depth, int device)
 {
-    if (v.stack != 24u) return v.stack;
+    if (v.stack != 24u || depth > 8u) return v.stack;
+    if (v.pool) return 32u;
     PathVariant v4 = v;
     v4.stack = 32u;
     const uint64_t resident4 = (uint64_t)persistent_grid(v4, device) * v.block;
-    if (v.pool) return depth <= 8u ? 32u : 24u;
-    if (depth <= 8u) return (uint64_t)total <= resident4 ? 64u : 32u;
-    return (uint64_t)total > 2u * resident4 ? 24u : 32u;
+    return (uint64_t)total <= resident4 ? 64u : 32u;
 }
 
 // The path kernel's launches for one frame.
